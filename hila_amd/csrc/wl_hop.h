@@ -62,26 +62,42 @@ __device__ __forceinline__ void hop_compute(cx<R> (&acc)[4][3], const HopBuf<R> 
     }
 }
 
-// Hop H = 2 mu + (0 forward, 1 backward): issue hop H+1's loads, then compute hop H.
-// nsp: neighbour element offsets of the spinor field (site index times the rhs count);
-// nl: neighbour site indices (backward links live at the neighbour); S: link block stride;
-// Ssp: spinor block stride; LF: stored entries per link (9, or 6 for two-row links).
-template <typename R, int SIGN, int H, bool NTL = true, int LF = 9>
+// The hop taken as the i-th: hop = 2 mu + (0 forward, 1 backward); t backward, x, y, z, t
+// forward.  Sweeping along t, the waves in flight span several time slices, and a slice's
+// spinors are read by those of the slice before (forward), its own (x, y, z) and those of the
+// slice after (backward).  With t backward first and t forward last these reads of one spinor
+// lie closest together in time, so more of them find it in the L2: the FP64 hop on 32^4 fetches
+// 796 MB instead of 860 (705 are needed), 135.2 us instead of 138.7 with t forward, t backward
+// at the end; M on 48^3 x 96 3156 us instead of 3208 (MI355X).
+__host__ __device__ constexpr int hop_order(int i) { return i == 0 ? 7 : i == 7 ? 6 : i - 1; }
+
+// Request the operands of hop H.  nsp: neighbour element offsets of the spinor field (site index
+// times the rhs count); nl: neighbour site indices (backward links live at the neighbour); S:
+// link block stride; Ssp: spinor block stride; LF: stored entries per link (9, or 6 for two-row
+// links).
+template <int H, bool NTL, int LF, typename R>
+__device__ __forceinline__ void hop_load_at(HopBuf<R> &b, const cx<R> *__restrict__ in, const cx<R> *gout,
+                                            const cx<R> *gin, int Ssp, int S, int k, const SiteNb &nsp,
+                                            const SiteNb &nl) {
+    constexpr int M = H / 2;
+    if constexpr (H % 2 == 0)
+        hop_load<NTL, LF>(b, in, gout + M * LF * S, Ssp, nsp.fwd[M], S, k);
+    else
+        hop_load<NTL, LF>(b, in, gin + M * LF * S, Ssp, nsp.bwd[M], S, nl.bwd[M]);
+}
+
+// The I-th hop of hop_order: issue the next one's loads, then compute this one.
+template <typename R, int SIGN, int I, bool NTL = true, int LF = 9>
 __device__ __forceinline__ void hop_chain(cx<R> (&acc)[4][3], HopBuf<R> (&buf)[2],
                                           const cx<R> *__restrict__ in, const cx<R> *gout,
                                           const cx<R> *gin, int Ssp, int S, int k,
                                           const SiteNb &nsp, const SiteNb &nl, R sf, R sb) {
-    if constexpr (H < 8) {
-        constexpr int HN = H + 1;
-        if constexpr (HN < 8) {
-            constexpr int MN = HN / 2;
-            if constexpr (HN % 2 == 0)
-                hop_load<NTL, LF>(buf[HN & 1], in, gout + MN * LF * S, Ssp, nsp.fwd[MN], S, k);
-            else
-                hop_load<NTL, LF>(buf[HN & 1], in, gin + MN * LF * S, Ssp, nsp.bwd[MN], S, nl.bwd[MN]);
-        }
-        hop_compute<H / 2, SIGN, (H % 2 == 0)>(acc, buf[H & 1], (H % 2 == 0) ? sf : sb);
-        hop_chain<R, SIGN, H + 1, NTL, LF>(acc, buf, in, gout, gin, Ssp, S, k, nsp, nl, sf, sb);
+    if constexpr (I < 8) {
+        if constexpr (I + 1 < 8)
+            hop_load_at<hop_order(I + 1), NTL, LF>(buf[(I + 1) & 1], in, gout, gin, Ssp, S, k, nsp, nl);
+        constexpr int H = hop_order(I);
+        hop_compute<H / 2, SIGN, (H % 2 == 0)>(acc, buf[I & 1], (H % 2 == 0) ? sf : sb);
+        hop_chain<R, SIGN, I + 1, NTL, LF>(acc, buf, in, gout, gin, Ssp, S, k, nsp, nl, sf, sb);
     }
 }
 
@@ -110,7 +126,7 @@ __device__ __forceinline__ void hop_sum(cx<R> (&acc)[4][3], const Geom &g, int k
 #pragma unroll
         for (int c = 0; c < 3; ++c) acc[s][c] = {R(0), R(0)};
     HopBuf<R> buf[2];
-    hop_load<NTL, LF>(buf[0], in, gout, S * N, nsp.fwd[0], S, k);
+    hop_load_at<hop_order(0), NTL, LF>(buf[0], in, gout, gin, S * N, S, k, nsp, n);
     hop_chain<R, SIGN, 0, NTL, LF>(acc, buf, in, gout, gin, S * N, S, k, nsp, n, sf, sb);
 }
 

@@ -196,24 +196,32 @@ __device__ __forceinline__ void rb_compute(cx<typename St<T>::R> (&acc)[NR][4][3
     }
 }
 
-// Hop H = 2 mu + (0 forward, 1 backward): issue hop H+1's loads, then compute hop H.
-template <typename T, int SIGN, int H, int NR, bool NTL, int LF>
+// Request the operands of hop H = 2 mu + (0 forward, 1 backward).
+template <int H, int NR, bool NTL, typename T, int LF>
+__device__ __forceinline__ void rb_load_at(RbBuf<T, NR> &b, const bool (&act)[NR],
+                                           const typename St<T>::E *__restrict__ in, size_t rs,
+                                           const typename St<T>::E *gout, const typename St<T>::E *gin, int S, int k,
+                                           const SiteNb &n) {
+    constexpr int M = H / 2;
+    if constexpr (H % 2 == 0)
+        rb_load<NR, NTL, T, LF>(b, act, in, rs, gout + M * LF * S, S, n.fwd[M], k);
+    else
+        rb_load<NR, NTL, T, LF>(b, act, in, rs, gin + M * LF * S, S, n.bwd[M], n.bwd[M]);
+}
+
+// The I-th hop of hop_order: issue the next one's loads, then compute this one.
+template <typename T, int SIGN, int I, int NR, bool NTL, int LF>
 __device__ __forceinline__ void rb_chain(cx<typename St<T>::R> (&acc)[NR][4][3], RbBuf<T, NR> (&buf)[2],
                                          const bool (&act)[NR], const typename St<T>::E *__restrict__ in,
                                          size_t rs, const typename St<T>::E *gout,
                                          const typename St<T>::E *gin, int S, int k, const SiteNb &n,
                                          typename St<T>::R sf, typename St<T>::R sb) {
-    if constexpr (H < 8) {
-        constexpr int HN = H + 1;
-        if constexpr (HN < 8) {
-            constexpr int MN = HN / 2;
-            if constexpr (HN % 2 == 0)
-                rb_load<NR, NTL, T, LF>(buf[HN & 1], act, in, rs, gout + MN * LF * S, S, n.fwd[MN], k);
-            else
-                rb_load<NR, NTL, T, LF>(buf[HN & 1], act, in, rs, gin + MN * LF * S, S, n.bwd[MN], n.bwd[MN]);
-        }
-        rb_compute<H / 2, SIGN, (H % 2 == 0), NR, T>(acc, buf[H & 1], act, (H % 2 == 0) ? sf : sb);
-        rb_chain<T, SIGN, H + 1, NR, NTL, LF>(acc, buf, act, in, rs, gout, gin, S, k, n, sf, sb);
+    if constexpr (I < 8) {
+        if constexpr (I + 1 < 8)
+            rb_load_at<hop_order(I + 1), NR, NTL, T, LF>(buf[(I + 1) & 1], act, in, rs, gout, gin, S, k, n);
+        constexpr int H = hop_order(I);
+        rb_compute<H / 2, SIGN, (H % 2 == 0), NR, T>(acc, buf[I & 1], act, (H % 2 == 0) ? sf : sb);
+        rb_chain<T, SIGN, I + 1, NR, NTL, LF>(acc, buf, act, in, rs, gout, gin, S, k, n, sf, sb);
     }
 }
 
@@ -331,9 +339,10 @@ __global__ __launch_bounds__(kBlock, 2) void k_dslash_rb(RbArgs<T> A) {
                 for (int c = 0; c < 3; ++c) acc[r][s][c] = {R(0), R(0)};
         if constexpr (PIPE) {
             RbBuf<T, NR> buf[2];
-            rb_load<NR, NTL, T, LF>(buf[0], act, in, rs, gout, S, n.fwd[0], k);
+            rb_load_at<hop_order(0), NR, NTL, T, LF>(buf[0], act, in, rs, gout, gin, S, k, n);
             rb_chain<T, SIGN, 0, NR, NTL, LF>(acc, buf, act, in, rs, gout, gin, S, k, n, sf, sb);
         } else {
+            rb_hop<3, SIGN, false, NR, NTL, T, LF>(acc, act, in, rs, gin + 3 * LF * S, S, n.bwd[3], n.bwd[3], sb);
             rb_hop<0, SIGN, true, NR, NTL, T, LF>(acc, act, in, rs, gout, S, n.fwd[0], k, R(1));
             rb_hop<0, SIGN, false, NR, NTL, T, LF>(acc, act, in, rs, gin, S, n.bwd[0], n.bwd[0], R(1));
             rb_hop<1, SIGN, true, NR, NTL, T, LF>(acc, act, in, rs, gout + LF * S, S, n.fwd[1], k, R(1));
@@ -341,7 +350,6 @@ __global__ __launch_bounds__(kBlock, 2) void k_dslash_rb(RbArgs<T> A) {
             rb_hop<2, SIGN, true, NR, NTL, T, LF>(acc, act, in, rs, gout + 2 * LF * S, S, n.fwd[2], k, R(1));
             rb_hop<2, SIGN, false, NR, NTL, T, LF>(acc, act, in, rs, gin + 2 * LF * S, S, n.bwd[2], n.bwd[2], R(1));
             rb_hop<3, SIGN, true, NR, NTL, T, LF>(acc, act, in, rs, gout + 3 * LF * S, S, n.fwd[3], k, sf);
-            rb_hop<3, SIGN, false, NR, NTL, T, LF>(acc, act, in, rs, gin + 3 * LF * S, S, n.bwd[3], n.bwd[3], sb);
         }
 
         rb_epilogue<T, EPI, NR>(A, acc, act, jf, k, nrm);
@@ -366,19 +374,21 @@ __device__ __forceinline__ void sp_load(RbBuf<T, NR> &b, const bool (&act)[NR],
         }
 }
 
-template <typename T, int SIGN, int H, int NR, bool PIPE>
+template <typename T, int SIGN, int I, int NR, bool PIPE>
 __device__ __forceinline__ void rb_chain_lds(cx<typename St<T>::R> (&acc)[NR][4][3], RbBuf<T, NR> (&buf)[2],
                                              const bool (&act)[NR], const typename St<T>::E *__restrict__ in,
                                              size_t rs, const typename St<T>::E *lu, int lane, int S,
                                              const SiteNb &n, typename St<T>::R sf, typename St<T>::R sb) {
     using R = typename St<T>::R;
-    if constexpr (H < 8) {
+    if constexpr (I < 8) {
+        constexpr int H = hop_order(I);
         if constexpr (PIPE) {
-            constexpr int HN = H + 1;
-            if constexpr (HN < 8)
-                sp_load<NR, T>(buf[HN & 1], act, in, rs, S, (HN % 2 == 0) ? n.fwd[HN / 2] : n.bwd[HN / 2]);
+            if constexpr (I + 1 < 8) {
+                constexpr int HN = hop_order(I + 1);
+                sp_load<NR, T>(buf[(I + 1) & 1], act, in, rs, S, (HN % 2 == 0) ? n.fwd[HN / 2] : n.bwd[HN / 2]);
+            }
         } else {
-            sp_load<NR, T>(buf[H & 1], act, in, rs, S, (H % 2 == 0) ? n.fwd[H / 2] : n.bwd[H / 2]);
+            sp_load<NR, T>(buf[I & 1], act, in, rs, S, (H % 2 == 0) ? n.fwd[H / 2] : n.bwd[H / 2]);
         }
         if constexpr (St<T>::scaled) {
             h2 ur[9];
@@ -387,14 +397,14 @@ __device__ __forceinline__ void rb_chain_lds(cx<typename St<T>::R> (&acc)[NR][4]
             const R sg = (H / 2 == 3) ? ((H % 2 == 0) ? sf : sb) : R(1);
 #pragma unroll
             for (int r = 0; r < NR; ++r)
-                if (act[r]) hop_pk<H / 2, SIGN, (H % 2 == 0)>(acc[r], buf[H & 1].w[r], ur, sg * buf[H & 1].sc[r]);
+                if (act[r]) hop_pk<H / 2, SIGN, (H % 2 == 0)>(acc[r], buf[I & 1].w[r], ur, sg * buf[I & 1].sc[r]);
         } else {
             cx<R> u[3][3];
 #pragma unroll
             for (int e = 0; e < 9; ++e) u[e / 3][e % 3] = widen(lu[(H * 9 + e) * 64 + lane]);
-            rb_compute_u<H / 2, SIGN, (H % 2 == 0), NR, T>(acc, buf[H & 1], u, act, (H % 2 == 0) ? sf : sb);
+            rb_compute_u<H / 2, SIGN, (H % 2 == 0), NR, T>(acc, buf[I & 1], u, act, (H % 2 == 0) ? sf : sb);
         }
-        rb_chain_lds<T, SIGN, H + 1, NR, PIPE>(acc, buf, act, in, rs, lu, lane, S, n, sf, sb);
+        rb_chain_lds<T, SIGN, I + 1, NR, PIPE>(acc, buf, act, in, rs, lu, lane, S, n, sf, sb);
     }
 }
 
@@ -457,7 +467,7 @@ __global__ __launch_bounds__(512, 1) void k_dslash_rb_lds(RbArgs<T> A) {
 #pragma unroll
                 for (int c = 0; c < 3; ++c) acc[r][s][c] = {R(0), R(0)};
         RbBuf<T, NR> buf[2];
-        if constexpr (PIPE) sp_load<NR, T>(buf[0], act, in, rs, S, n.fwd[0]);
+        if constexpr (PIPE) sp_load<NR, T>(buf[0], act, in, rs, S, n.bwd[3]);
         rb_chain_lds<T, SIGN, 0, NR, PIPE>(acc, buf, act, in, rs, lu, lane, S, n, sf, sb);
         rb_epilogue<T, EPI, NR>(A, acc, act, jf, k, nrm);
     }
