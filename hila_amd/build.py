@@ -22,14 +22,15 @@ BUILD = os.path.join(ROOT, "hila_amd", "_build")
 LIBDIR = os.path.join(ROOT, "hila_amd", "lib")
 LIB = os.path.join(LIBDIR, "libhila_wilson.so")
 
-HIP_SOURCES = ["wl_rb_f16.hip", "wl_rb_f32.hip", "wl_rb_f32r.hip", "wl_rb_f64.hip", "wl_rb_f64r.hip",
+HIP_SOURCES = ["wl_rb_f16.hip", "wl_tile_f16.hip", "wl_rb_f32.hip", "wl_rb_f32r.hip", "wl_rb_f64.hip", "wl_rb_f64r.hip",
                "wl_dslash.hip", "wl_multi.hip",
                "wl_blas.hip", "wl_api.hip", "wl_cg.hip", "wl_cgp.hip", "wl_bcg.hip", "wl_noalloc.hip", "wl_serve.hip", "wl_config.hip", "wl_mre.hip", "wl_force.hip"]
 # Per-source device flags.  wl_rb_f16.hip: without the v_dot2c_f32_f16 encoding (dot5-insts,
 # which accumulates in place and so needs a zero move to start every FP16 dot-product chain)
 # the compiler selects v_dot2_f32_f16, whose accumulator is a separate operand (an inline 0 at
 # the start of a chain): 10% fewer VALU instructions in the FP16 hopping kernels.
-SOURCE_FLAGS = {"wl_rb_f16.hip": ["-Xclang", "-target-feature", "-Xclang", "-dot5-insts"]}
+_NO_DOT2C = ["-Xclang", "-target-feature", "-Xclang", "-dot5-insts"]
+SOURCE_FLAGS = {"wl_rb_f16.hip": _NO_DOT2C, "wl_tile_f16.hip": _NO_DOT2C}
 # C++ programs written against the HILA-style mirror (include/hila_wilson.hpp)
 CPP_TESTS = [os.path.join(ROOT, "tests", "cpp", "test_wilson_evenodd.cpp")]
 CPP_TEST_BUILD = os.path.join(ROOT, "tests", "cpp", "_build")

@@ -343,6 +343,23 @@ Geom mr_geom(const wl_ctx *c, int prec, int nb, int nr, bool lds_links) {
     return g;
 }
 
+// Right-hand sides per workgroup of the LDS-tiled kernel (wl_tile.h) for N of them, 0: the
+// lane-per-site kernel.  A tile's links and first rhs are loaded with nothing to overlap them
+// (31 us of a launch on 32^4, 14 us for each rhs), so it takes six: M in FP16, us per rhs, lane
+// per site / tiled (MI355X): 24^3x48 4 rhs 30.8 / 32.4, 6 rhs 29.7 / 28.6, 12 rhs 28.9 / 25.2;
+// 32^4 12 rhs 45.0 / 35.5; 16^3x32 12 rhs 5.8 / 5.2.  The rhs are split into as many groups, of
+// three at least, as make 1024 workgroups (20^4 with 320 tiles, 12 rhs: 7.35 in one group, 6.89
+// in four; 24^4 with 864: 14.4 and 13.2 in two); with fewer than 256 tiles (16^4, 12 rhs: 3.06 / 3.15)
+// and where tiles waste more than one lane in eight (48^3x24, rows of 24: 119 / 121) it does not
+// pay.  Not where the caller chose a shape for the lane-per-site kernel, as wl_autotune does.
+int tile_rhs(const wl_ctx *c, int prec, int N) {
+    const TileGeom &t = c->tile;
+    if (prec != WL_F16 || N < 6 || t.tiles < 256 || (int64_t)t.tiles * t.nt * 8 > (int64_t)c->g.vh * 9) return 0;
+    if (c->rhs_block || c->rhs_launch || c->link_load || c->pipeline || !c->blk_auto || !c->lds_auto) return 0;
+    const int groups = std::min((1024 + t.tiles - 1) / t.tiles, N / 3);
+    return (N + groups - 1) / groups;
+}
+
 int dslash_mr_all(wl_ctx *c, int prec, void *out, int out_par, const void *in, const void *xin,
                   double a, int sign, int epi, int N, const int *all_done, CgState *st, void *x,
                   const void *p, void *r, int *pstride_out) {
@@ -352,6 +369,31 @@ int dslash_mr_all(wl_ctx *c, int prec, void *out, int out_par, const void *in, c
         if (rc) return rc;
     }
     if (!gauge_for(c, prec)) return fail(WL_E_STATE, "links of precision %d not prepared (ensure_gauge)", prec);
+    if (const int per = tile_rhs(c, prec, N)) {
+        if (epi == EPI_AXPY_NORM || epi == EPI_CGUPD)
+            if (int rc = ensure_partials(c, (size_t)N * tile_slots(c->tile))) return rc;
+        MrLaunch L{};
+        L.out = out;
+        L.in = in;
+        L.xin = xin;
+        L.gauge = gauge_for(c, prec);
+        L.a = a;
+        L.b = 1.0 + c->op_shift;
+        L.out_par = out_par;
+        L.sign = sign;
+        L.epi = epi;
+        L.NB = N;
+        L.NR = per;
+        L.all_done = all_done;
+        L.st = st;
+        L.x = x;
+        L.p = p;
+        L.r = r;
+        L.partials = c->partials;
+        HIPCHK(launch_dslash_tile(c->g, c->tile, L, c->stream));
+        if (pstride_out) *pstride_out = tile_slots(c->tile);
+        return WL_OK;
+    }
     const int nr = rhs_per_lane(c, prec, N);
     const int nl = rhs_per_launch(c, nr, N);
     for (int j0 = 0; j0 < N; j0 += nl) {
@@ -514,6 +556,7 @@ extern "C" int wl_create(const int dims[4], int antiperiodic_t, int device, wl_c
     c->g.blk = dslash_block_auto(c->g.vh);
     c->g.dir = dir_auto(c->g.vh);
     (void)set_chunk(c->g, -1);
+    c->tile = tile_geom(c->g);
     DeviceGuard dg(device);
     int rc = WL_OK;
     // one partial-sum slot per workgroup of the largest grid (64-lane workgroups)

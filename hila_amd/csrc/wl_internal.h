@@ -135,6 +135,60 @@ struct MrLaunch {
     void *r;
     double *partials;
 };
+// Tiles of the LDS-tiled FP16 hopping kernel (wl_tile.h): ty x tz rows (a row: all x) of one time
+// slice.  An LDS buffer holds a tile's rows and the rows around it, corners included, as a
+// (ty + 2) x (tz + 2) grid of rows: at most kTileSites sites (two buffers are then 60 KB, and
+// two workgroups share a CU); a thread stages kTileStage sites of it at most.
+constexpr int kTileSites = 576;
+constexpr int kTileStage = 2;
+struct TileGeom {
+    int ty, tz;  // rows of a tile in y and in z
+    int ny, nz;  // tiles of a time slice in y and in z
+    int zs;      // z tiles of a slab: the tiles of a slab are swept along t together
+    int lanes;   // output sites of a whole tile
+    int nt;      // threads of a workgroup
+    int tiles;   // tiles of a parity; 0: the lattice has no such tiling
+    int per;     // rhs of a workgroup
+};
+// The tiling of the LDS-tiled kernel with the least work per site: arithmetic of the lanes, idle
+// ones too (about 12 clocks of a CU per site and rhs; 5% more where the 8 waves that a CU holds
+// are no whole number of workgroups), and staged sites (1.6).  On 24^3 slices 4x4 and 5x4 rows
+// time within 2% of it, 7x3 5% and 3x7 10% slower; on 32^3 4x4 is 15% faster than 3x5 and 2x7.
+// Slabs of up to 8 tiles of a slice are swept along t: 64 workgroups of an XCD then span 8 or
+// more slices, and share what they read in y, z and t (32^3: 35.5 us for slabs of 8 tiles, 36.5
+// and 38.4 for 16 and 32).
+inline TileGeom tile_geom(const Geom &g) {
+    const int Xh = g.L[0] / 2, Ly = g.L[1], Lz = g.L[2];
+    TileGeom best{};
+    if (g.stride > 1 << 26) return best;  // an rhs block is addressed with 32-bit byte offsets
+    double best_cost = 1e300;
+    for (int ty = 1; ty <= Ly && ty * Xh <= 256; ++ty)
+        for (int tz = 1; tz <= Lz && ty * tz * Xh <= 256; ++tz) {
+            TileGeom t{};
+            t.ty = ty;
+            t.tz = tz;
+            t.lanes = ty * tz * Xh;
+            t.nt = (t.lanes + 63) / 64 * 64;
+            const int stage = (ty * tz + 2 * ty + 2 * tz) * Xh;
+            if ((ty + 2) * (tz + 2) * Xh > kTileSites || stage > kTileStage * t.nt) continue;
+            t.ny = (Ly + ty - 1) / ty;
+            t.nz = (Lz + tz - 1) / tz;
+            const double sites = (double)Xh * Ly * Lz, n = (double)t.ny * t.nz;
+            const int waves = t.nt / 64;
+            const double cost = n * t.nt / sites * 12.0 * (8 / waves * waves < 8 ? 1.05 : 1.0) + n * stage / sites * 1.6;
+            if (cost >= best_cost) continue;
+            best_cost = cost;
+            t.tiles = t.ny * t.nz * g.L[3];
+            t.zs = 1;
+            for (int s = 1; s <= t.nz; ++s)
+                if (t.nz % s == 0 && (s == 1 || s * t.ny <= 8)) t.zs = s;
+            best = t;
+        }
+    return best;
+}
+// partial sums per rhs of a launch: one for each wave of each tile
+inline int tile_slots(const TileGeom &t) { return t.tiles * (t.nt / 64); }
+hipError_t launch_dslash_tile(const Geom &g, const TileGeom &tg, const MrLaunch &L, hipStream_t s);
 hipError_t launch_dslash_mr(int prec, const Geom &g, const MrLaunch &L, hipStream_t s);
 int mr_segments(const Geom &g);
 hipError_t launch_finish_mr(double *partials, int pstride, int n, int N, CgState *st,
@@ -191,6 +245,7 @@ struct wl_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     wl::Geom g{};
+    wl::TileGeom tile{};
     int64_t V = 0;
     int antiperiodic = 1;
     void *gauge64 = nullptr;
