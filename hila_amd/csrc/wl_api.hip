@@ -361,8 +361,8 @@ int tile_rhs(const wl_ctx *c, int prec, int N) {
 }
 
 int dslash_mr_all(wl_ctx *c, int prec, void *out, int out_par, const void *in, const void *xin,
-                  double a, int sign, int epi, int N, const int *all_done, CgState *st, void *x,
-                  const void *p, void *r, int *pstride_out) {
+                  double a, int sign, int epi, int N, const int *all_done, CgState *st, void *r,
+                  int *pstride_out) {
     const int pstride = mr_segments(c->g);
     if (epi == EPI_AXPY_NORM || epi == EPI_CGUPD) {
         int rc = ensure_partials(c, (size_t)N * pstride);
@@ -386,8 +386,6 @@ int dslash_mr_all(wl_ctx *c, int prec, void *out, int out_par, const void *in, c
         L.NR = per;
         L.all_done = all_done;
         L.st = st;
-        L.x = x;
-        L.p = p;
         L.r = r;
         L.partials = c->partials;
         HIPCHK(launch_dslash_tile(c->g, c->tile, L, c->stream));
@@ -418,8 +416,6 @@ int dslash_mr_all(wl_ctx *c, int prec, void *out, int out_par, const void *in, c
         L.pipe = c->pipeline == 0;
         L.all_done = all_done;
         L.st = st;
-        L.x = x;
-        L.p = p;
         L.r = r;
         L.partials = c->partials;
         HIPCHK(launch_dslash_mr(prec, mr_geom(c, prec, L.NB, L.NR, L.lds_links), L, c->stream));
@@ -431,10 +427,9 @@ int dslash_mr_all(wl_ctx *c, int prec, void *out, int out_par, const void *in, c
 int meo_mr(wl_ctx *c, int prec, void *out, const void *in, void *t, double kappa, int sign,
            int epi2, int N, const int *all_done, CgState *st, int *pstride_out) {
     int rc = dslash_mr_all(c, prec, t, 1, in, nullptr, -kappa, sign, EPI_SET, N, all_done, st,
-                           nullptr, nullptr, nullptr, nullptr);
+                           nullptr, nullptr);
     if (rc) return rc;
-    return dslash_mr_all(c, prec, out, 0, t, in, kappa, sign, epi2, N, all_done, st, nullptr,
-                         nullptr, nullptr, pstride_out);
+    return dslash_mr_all(c, prec, out, 0, t, in, kappa, sign, epi2, N, all_done, st, nullptr, pstride_out);
 }
 
 int field_upload_async(wl_ctx *c, void *data, int prec, int N, int j, const double *host) {
@@ -765,7 +760,7 @@ extern "C" int wl_dslash_eo(wl_ctx *c, wl_field *out, const wl_field *in, double
         return dslash_one(c, in->prec, out->data, out_par, in->data, nullptr, -kappa, sign, EPI_SET,
                           nullptr, FIN_NONE);
     return dslash_mr_all(c, in->prec, out->data, out_par, in->data, nullptr, -kappa, sign, EPI_SET,
-                         in->nrhs, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
+                         in->nrhs, nullptr, nullptr, nullptr, nullptr);
 }
 
 namespace {
@@ -969,7 +964,7 @@ int time_hop_mr(wl_ctx *c, int prec, void *out, const void *in, int N, int iters
     for (int i = 0; i < 2 + iters; ++i) {
         if (i == 2) HIPCHK(hipEventRecord(e0, c->stream));
         if (int rc = dslash_mr_all(c, prec, out, 1, in, nullptr, -0.125, 1, EPI_SET, N, nullptr, nullptr, nullptr,
-                                   nullptr, nullptr, nullptr))
+                                   nullptr))
             return rc;
     }
     HIPCHK(hipEventRecord(e1, c->stream));

@@ -34,17 +34,44 @@ __device__ __forceinline__ double site_cg_init(const cx<double> *__restrict__ b,
     return s;
 }
 
-// p = beta p + r at site k (conjugate_gradient.h:94)
-template <typename R>
-__device__ __forceinline__ void site_xpay(cx<R> *__restrict__ p, const cx<R> *__restrict__ r, R beta, int S, int k) {
-    cx<R> pv[4][3], rv[4][3];
-    ld_site<R>(p, S, k, pv);
-    ld_site<R>(r, S, k, rv);
+// out = beta p + r at site k (conjugate_gradient.h:94), p given; one rhs of a storage T
+template <typename T>
+__device__ __forceinline__ void site_xpay(typename St<T>::E *out, cx<typename St<T>::R> (&pv)[4][3],
+                                          const typename St<T>::E *__restrict__ r, typename St<T>::R beta, int S,
+                                          int k) {
+    cx<typename St<T>::R> rv[4][3];
+    ld_site<T>(r, S, k, rv);
 #pragma unroll
     for (int s = 0; s < 4; ++s)
 #pragma unroll
         for (int c = 0; c < 3; ++c) pv[s][c] = beta * pv[s][c] + rv[s][c];
-    st_site<R>(p, S, k, pv);
+    st_site<T>(out, S, k, pv);
+}
+template <typename R>
+__device__ __forceinline__ void site_xpay(cx<R> *p, const cx<R> *__restrict__ r, R beta, int S, int k) {
+    cx<R> pv[4][3];
+    ld_site<R>(p, S, k, pv);
+    site_xpay<R>(p, pv, r, beta, S, k);
+}
+
+// The ring slots of a solve (PRing) and what a launch does with them: x += alpha_m p_m of slots
+// 0 .. n - 1 at site k, in order, into x in arithmetic A; pv returns the last slot's p.
+template <typename T>
+struct RingArgs {
+    typename St<T>::E *p[kRing];
+};
+template <typename T, typename A>
+__device__ __forceinline__ void site_ring(cx<A> *x, const RingArgs<T> &ring, const double *alphas, int n, size_t off,
+                                          int S, int k, cx<typename St<T>::R> (&pv)[4][3]) {
+    cx<A> xv[4][3];
+    ld_site<A, true>(x, S, k, xv);
+#pragma unroll
+    for (int m = 0; m < kRing; ++m)
+        if (m < n) {
+            ld_site<T>(ring.p[m] + off, S, k, pv);
+            x_add<typename St<T>::R>(xv, (A)alphas[m], pv);
+        }
+    st_site<A, true>(x, S, k, xv);
 }
 
 // ||b(k) - v(k)||^2 (FP64)

@@ -171,14 +171,44 @@ __global__ __launch_bounds__(kBlock) void k_cg_init(const cx<double> *__restrict
     reduce_partial(s, ra);
 }
 
-template <typename R>
-__global__ __launch_bounds__(kBlock) void k_cg_xpay(cx<R> *__restrict__ p,
-                                                    const cx<R> *__restrict__ r,
+// Next p = beta p + r from one ring slot to another (or in place); X (the ring is full): after
+// x += alpha p of its n slots, `from` the last of them.
+template <typename R, bool X>
+__global__ __launch_bounds__(kBlock) void k_cg_xpay(const cx<R> *from, cx<R> *to, const cx<R> *__restrict__ r,
+                                                    RingArgs<R> ring, int n, cx<double> *__restrict__ x,
                                                     const CgState *st, int vh, int S) {
     if (st->done) return;
     const int k = blockIdx.x * kBlock + threadIdx.x;
     if (k >= vh) return;
+    cx<R> pv[4][3];
+    if constexpr (X)
+        site_ring<R, double>(x, ring, st->alphas, n, 0, S, k, pv);
+    else
+        ld_site<R>(from, S, k, pv);
+    site_xpay<R>(to, pv, r, (R)st->beta, S, k);
+}
+
+// p = beta p + r in place
+template <typename R>
+__global__ __launch_bounds__(kBlock) void k_cg_restart(cx<R> *__restrict__ p, const cx<R> *__restrict__ r,
+                                                       const CgState *st, int vh, int S) {
+    if (st->done) return;
+    const int k = blockIdx.x * kBlock + threadIdx.x;
+    if (k >= vh) return;
     site_xpay<R>(p, r, (R)st->beta, S, k);
+}
+
+// x += alpha p of the slots that a stopped or paused solve has pending; its last p to slot 0
+template <typename R>
+__global__ __launch_bounds__(kBlock) void k_cg_flush(RingArgs<R> ring, cx<double> *__restrict__ x, const CgState *st,
+                                                     int vh, int S) {
+    const int n = st->done ? st->pend : 0;
+    if (n == 0) return;
+    const int k = blockIdx.x * kBlock + threadIdx.x;
+    if (k >= vh) return;
+    cx<R> pv[4][3];
+    site_ring<R, double>(x, ring, st->alphas, n, 0, S, k, pv);
+    if (n > 1) st_site<R>(ring.p[0], S, k, pv);
 }
 
 // p = beta p + r of the launch-folded CG iteration `it` (0-based), with the finish kernel's
@@ -187,9 +217,12 @@ __global__ __launch_bounds__(kBlock) void k_cg_xpay(cx<R> *__restrict__ p,
 // rrnew / rr_it, and updates p unless the solve has ended; workgroup 0 records the state
 // (rrnew, iter, done; beta and rr, with rr_(it+1) in slot (it + 1) & 1, unless converged).
 // The done flag is read once per workgroup: workgroup 0 may set it meanwhile, and p is not
-// needed once it is set.
-__global__ __launch_bounds__(kBlock) void k_cg_xpay_fold(cx<double> *__restrict__ p,
-                                                         const cx<double> *__restrict__ r, CgState *st,
+// needed once it is set (the solution then gets the pending slots from launch_cg_flush).  Slots
+// and X as in k_cg_xpay.
+template <bool X>
+__global__ __launch_bounds__(kBlock) void k_cg_xpay_fold(const cx<double> *from, cx<double> *to,
+                                                         const cx<double> *__restrict__ r, RingArgs<double> ring,
+                                                         int nring, cx<double> *__restrict__ x, CgState *st,
                                                          const double *parts, int n, int it, int vh, int S) {
     __shared__ int ended;
     if (threadIdx.x == 0) ended = st->done;
@@ -214,7 +247,13 @@ __global__ __launch_bounds__(kBlock) void k_cg_xpay_fold(cx<double> *__restrict_
     }
     if (conv || iter >= st->maxiters) return;
     const int k = blockIdx.x * kBlock + threadIdx.x;
-    if (k < vh) site_xpay<double>(p, r, beta, S, k);
+    if (k >= vh) return;
+    cx<double> pv[4][3];
+    if constexpr (X)
+        site_ring<double, double>(x, ring, st->alphas, nring, 0, S, k, pv);
+    else
+        ld_site<double>(from, S, k, pv);
+    site_xpay<double>(to, pv, r, beta, S, k);
 }
 
 // Reliable update: r = b - DDp in FP64 (DDp = M^dag M x in FP64), stored in the inner
@@ -295,10 +334,24 @@ __global__ __launch_bounds__(kBlock) void k_finish(RedArgs ra, int n, int fin, c
 
 // ------------------------------------------------------------------- launchers ---------
 
-hipError_t launch_cg_xpay_fold(const Geom &g, void *p, const void *r, CgState *st, const double *parts, int n,
-                               int it, hipStream_t s) {
-    hipLaunchKernelGGL(k_cg_xpay_fold, dim3(nblocks(g)), dim3(kBlock), 0, s, (cx<double> *)p, (const cx<double> *)r,
-                       st, parts, n, it, g.vh, g.stride);
+template <typename T>
+static RingArgs<T> ring_args(const PRing &ring) {
+    RingArgs<T> a;
+    for (int m = 0; m < kRing; ++m) a.p[m] = (typename St<T>::E *)(m < ring.n ? ring.p[m] : nullptr);
+    return a;
+}
+
+hipError_t launch_cg_xpay_fold(const Geom &g, const PRing &ring, const void *r, void *x, CgState *st,
+                               const double *parts, int n, int it, hipStream_t s) {
+    const int q = it % ring.n, to = (q + 1) % ring.n;
+    if (ring.n > 1 && to == 0)
+        hipLaunchKernelGGL(k_cg_xpay_fold<true>, dim3(nblocks(g)), dim3(kBlock), 0, s, (const cx<double> *)ring.p[q], (cx<double> *)ring.p[to],
+                           (const cx<double> *)r, ring_args<double>(ring), ring.n, (cx<double> *)x, st, parts, n, it,
+                           g.vh, g.stride);
+    else
+        hipLaunchKernelGGL(k_cg_xpay_fold<false>, dim3(nblocks(g)), dim3(kBlock), 0, s, (const cx<double> *)ring.p[q], (cx<double> *)ring.p[to],
+                           (const cx<double> *)r, ring_args<double>(ring), ring.n, (cx<double> *)x, st, parts, n, it,
+                           g.vh, g.stride);
     return hipGetLastError();
 }
 
@@ -405,14 +458,50 @@ hipError_t launch_cg_init(const Geom &g, const void *b, const void *DDp, void *r
     return e != hipSuccess ? e : launch_finish(ra, nblocks(g), FIN_RR, nullptr, s);
 }
 
-hipError_t launch_cg_xpay(int prec, const Geom &g, void *p, const void *r, const CgState *st,
-                          hipStream_t s) {
+template <typename R>
+static void xpay_t(const Geom &g, const PRing &ring, int q, const void *r, void *x, const CgState *st, hipStream_t s) {
+    const int to = (q + 1) % ring.n;
+    if (ring.n > 1 && to == 0)
+        hipLaunchKernelGGL((k_cg_xpay<R, true>), grid_sites(g), dim3(kBlock), 0, s, (const cx<R> *)ring.p[q],
+                           (cx<R> *)ring.p[to], (const cx<R> *)r, ring_args<R>(ring), ring.n, (cx<double> *)x, st,
+                           g.vh, g.stride);
+    else
+        hipLaunchKernelGGL((k_cg_xpay<R, false>), grid_sites(g), dim3(kBlock), 0, s, (const cx<R> *)ring.p[q],
+                           (cx<R> *)ring.p[to], (const cx<R> *)r, ring_args<R>(ring), ring.n, (cx<double> *)x, st,
+                           g.vh, g.stride);
+}
+
+hipError_t launch_cg_xpay(int prec, const Geom &g, const PRing &ring, int q, const void *r, void *x,
+                          const CgState *st, hipStream_t s) {
     if (prec == WL_F64)
-        hipLaunchKernelGGL(k_cg_xpay<double>, grid_sites(g), dim3(kBlock), 0, s, (cx<double> *)p,
+        xpay_t<double>(g, ring, q, r, x, st, s);
+    else if (prec == WL_F32)
+        xpay_t<float>(g, ring, q, r, x, st, s);
+    else
+        return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+hipError_t launch_cg_restart(int prec, const Geom &g, void *p, const void *r, const CgState *st, hipStream_t s) {
+    if (prec == WL_F64)
+        hipLaunchKernelGGL(k_cg_restart<double>, grid_sites(g), dim3(kBlock), 0, s, (cx<double> *)p,
                            (const cx<double> *)r, st, g.vh, g.stride);
     else if (prec == WL_F32)
-        hipLaunchKernelGGL(k_cg_xpay<float>, grid_sites(g), dim3(kBlock), 0, s, (cx<float> *)p,
+        hipLaunchKernelGGL(k_cg_restart<float>, grid_sites(g), dim3(kBlock), 0, s, (cx<float> *)p,
                            (const cx<float> *)r, st, g.vh, g.stride);
+    else
+        return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+hipError_t launch_cg_flush(int prec, const Geom &g, const PRing &ring, void *x, const CgState *st, hipStream_t s) {
+    if (ring.n == 1) return hipSuccess;
+    if (prec == WL_F64)
+        hipLaunchKernelGGL(k_cg_flush<double>, grid_sites(g), dim3(kBlock), 0, s, ring_args<double>(ring),
+                           (cx<double> *)x, st, g.vh, g.stride);
+    else if (prec == WL_F32)
+        hipLaunchKernelGGL(k_cg_flush<float>, grid_sites(g), dim3(kBlock), 0, s, ring_args<float>(ring),
+                           (cx<double> *)x, st, g.vh, g.stride);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();

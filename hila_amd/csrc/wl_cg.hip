@@ -38,6 +38,8 @@ int cg_f64(wl_ctx *c, const CgWork &w, void *x, size_t x_bytes, const void *b, d
     const auto t0 = std::chrono::steady_clock::now();
     int rc;
     void *r = w.r, *p = w.p, *Dp = w.Dp, *DDp = w.DDp, *t = w.t;
+    // DDp is free between the initial and the true residual
+    const PRing ring{{p, DDp}, c->g.dir ? 1 : 2};
     const RedArgs ra = red_args(w);
     const int *done = &w.st->done;
     const bool fold = cg_fold(c, w);
@@ -79,10 +81,13 @@ int cg_f64(wl_ctx *c, const CgWork &w, void *x, size_t x_bytes, const void *b, d
     while (!done_h && enqueued < maxiters) {
         const int n = std::min(kChunk, maxiters - enqueued);
         for (int it = 0; it < n; ++it) {
+            RedArgs rs = ra;
+            rs.slot = (enqueued + it) % ring.n;
+            void *ps = ring.p[rs.slot];
             // Dp = M p, pDp = |Dp|^2, alpha = rr / pDp (folded: alpha in the update pass)
-            if ((rc = meo_one(c, ra, WL_F64, Dp, p, t, kappa, +1, EPI_AXPY_NORM, done, fold ? FIN_NONE : FIN_ALPHA)))
+            if ((rc = meo_one(c, rs, WL_F64, Dp, ps, t, kappa, +1, EPI_AXPY_NORM, done, fold ? FIN_NONE : FIN_ALPHA)))
                 return rc;
-            // DDp = M^dag Dp fused with x += alpha p, r -= alpha DDp, rrnew = |r|^2, test, beta
+            // DDp = M^dag Dp fused with r -= alpha DDp, rrnew = |r|^2, test, beta
             if ((rc = dslash_one(c, ra, WL_F64, t, 1, Dp, nullptr, -kappa, -1, EPI_SET, done, FIN_NONE)))
                 return rc;
             DslashLaunch L{};
@@ -96,12 +101,12 @@ int cg_f64(wl_ctx *c, const CgWork &w, void *x, size_t x_bytes, const void *b, d
             L.b = 1.0 + c->op_shift;
             L.out_par = 0;
             L.sign = -1;
-            L.epi = EPI_CGUPD;
+            L.epi = ring.n == 1 ? EPI_CGUPDX : EPI_CGUPD;
             L.done = done;
             L.x = x;
             L.p = p;
             L.r = r;
-            L.red = ra;
+            L.red = rs;
             L.fin = FIN_RRNEW;
             if (fold) {
                 L.red.partials = parts2;
@@ -111,11 +116,11 @@ int cg_f64(wl_ctx *c, const CgWork &w, void *x, size_t x_bytes, const void *b, d
                 L.fold_it = enqueued + it;
             }
             HIPCHK(launch_dslash(WL_F64, c->g, L, c->stream));
-            // p = beta p + r (folded: with the convergence test and beta)
+            // p = beta p + r, and x of a full ring (folded: with the convergence test and beta)
             if (fold)
-                HIPCHK(launch_cg_xpay_fold(c->g, p, r, w.st, parts2, nhop, enqueued + it, c->stream));
+                HIPCHK(launch_cg_xpay_fold(c->g, ring, r, x, w.st, parts2, nhop, enqueued + it, c->stream));
             else
-                HIPCHK(launch_cg_xpay(WL_F64, c->g, p, r, w.st, c->stream));
+                HIPCHK(launch_cg_xpay(WL_F64, c->g, ring, rs.slot, r, x, w.st, c->stream));
         }
         enqueued += n;
         HIPCHK(hipMemcpyAsync(&c->st_host->done, &w.st->done, sizeof(int), hipMemcpyDeviceToHost, c->stream));
@@ -123,6 +128,7 @@ int cg_f64(wl_ctx *c, const CgWork &w, void *x, size_t x_bytes, const void *b, d
         done_h = c->st_host->done;
     }
 
+    HIPCHK(launch_cg_flush(WL_F64, c->g, ring, x, w.st, c->stream));
     // true residual |b - M^dag M x|^2 recomputed in FP64
     if ((rc = meo_one(c, ra, WL_F64, Dp, x, t, kappa, +1, EPI_AXPY, nullptr, FIN_NONE))) return rc;
     if ((rc = meo_one(c, ra, WL_F64, DDp, Dp, t, kappa, -1, EPI_AXPY, nullptr, FIN_NONE))) return rc;
@@ -172,6 +178,9 @@ int cg_mixed(wl_ctx *c, void *x, const void *b, double kappa, double accuracy, i
     if ((rc = ensure_tmp(c, prec, todd, WL_ODD))) return rc;
     void *r = c->mx_r->data, *p = c->mx_p->data, *Dp = c->mx_Dp->data, *t = (*todd)->data;
     void *Dp64 = c->cg_Dp->data, *DDp64 = c->cg_DDp->data, *t64 = c->tmp_odd64->data;
+    // the FP64 fields are free between reliable updates (with an FP64 inner precision t64 is not)
+    const PRing ring{{p, DDp64, Dp64, t64}, c->g.dir ? 1 : prec == WL_F64 ? 2 : 4};
+    static_assert(kChunk % 4 == 0, "a chunk ends with an empty ring");
     const RedArgs ra = red_args(c);
     const int *done = &c->st->done;
 
@@ -184,9 +193,10 @@ int cg_mixed(wl_ctx *c, void *x, const void *b, double kappa, double accuracy, i
     HIPCHK(hipMemcpyAsync(c->st, c->st_host, sizeof(CgState), hipMemcpyHostToDevice, c->stream));
     HIPCHK(launch_norm2(WL_F64, c->g, b, 1, 0, ra, FIN_SOURCE, nullptr, c->stream));
 
-    // reliable update: r = b - M^dag M x in FP64, r_lo = r, restart (or converged)
+    // reliable update: what x lacks, r = b - M^dag M x in FP64, r_lo = r, restart (or converged)
     auto reliable_update = [&]() -> int {
         int e;
+        HIPCHK(launch_cg_flush(prec, c->g, ring, x, c->st, c->stream));
         if ((e = meo_one(c, WL_F64, Dp64, x, t64, kappa, +1, EPI_AXPY, nullptr, FIN_NONE))) return e;
         if ((e = meo_one(c, WL_F64, DDp64, Dp64, t64, kappa, -1, EPI_AXPY, nullptr, FIN_NONE))) return e;
         HIPCHK(launch_residual_update(prec, c->g, b, DDp64, r, ra, c->stream));
@@ -213,10 +223,13 @@ int cg_mixed(wl_ctx *c, void *x, const void *b, double kappa, double accuracy, i
     while (done_h == 0 || done_h == 3 || done_h == 4) {
         if (done_h == 3 || done_h == 4) {
             if ((rc = reliable_update())) return rc;
-            HIPCHK(launch_cg_xpay(prec, c->g, p, r, c->st, c->stream));  // skipped if converged
+            HIPCHK(launch_cg_restart(prec, c->g, p, r, c->st, c->stream));  // skipped if converged
         }
         for (int it = 0; it < kChunk; ++it) {
-            if ((rc = meo_one(c, prec, Dp, p, t, kappa, +1, EPI_AXPY_NORM, done, FIN_ALPHA))) return rc;
+            RedArgs rs = ra;
+            rs.slot = it % ring.n;
+            if ((rc = meo_one(c, rs, prec, Dp, ring.p[rs.slot], t, kappa, +1, EPI_AXPY_NORM, done, FIN_ALPHA)))
+                return rc;
             if ((rc = dslash_one(c, prec, t, 1, Dp, nullptr, -kappa, -1, EPI_SET, done, FIN_NONE)))
                 return rc;
             DslashLaunch L{};
@@ -229,15 +242,15 @@ int cg_mixed(wl_ctx *c, void *x, const void *b, double kappa, double accuracy, i
             L.b = 1.0 + c->op_shift;
             L.out_par = 0;
             L.sign = -1;
-            L.epi = EPI_CGUPD;
+            L.epi = ring.n == 1 ? EPI_CGUPDX : EPI_CGUPD;
             L.done = done;
             L.x = x;
             L.p = p;
             L.r = r;
-            L.red = ra;
+            L.red = rs;
             L.fin = FIN_RRNEW_MIXED;
             HIPCHK(launch_dslash(prec, c->g, L, c->stream));
-            HIPCHK(launch_cg_xpay(prec, c->g, p, r, c->st, c->stream));
+            HIPCHK(launch_cg_xpay(prec, c->g, ring, rs.slot, r, x, c->st, c->stream));
         }
         HIPCHK(hipMemcpyAsync(&c->st_host->done, &c->st->done, sizeof(int), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(hipEventRecord(ev, c->stream));
@@ -373,6 +386,8 @@ int BatchCG::begin(wl_ctx *c, void *x, const void *b, int N, const CgSpec &spec)
         if ((rc = work_field(c, W_Y, WL_F32, WL_EVEN, N, &Y_))) return rc;
         acc_ = Y_->data;
     }
+    // the FP64 work fields are free between true residuals, and no smaller than P_
+    ring_ = PRing{{P_->data, DDP64_->data, DP64_->data, T64_->data}, 4};
     pplain_ = nblocks(c->g);
     cap_chunks_ = s_.maxiters > 0 ? (s_.maxiters + kChunk - 1) / kChunk + 4 : 0;
 
@@ -423,22 +438,23 @@ int BatchCG::enqueue_chunk_body(int slot) {
     int rc;
     for (int it = 0; it < kChunk; ++it) {
         int ps = 0;
+        const int q = it % ring_.n;
         // Dp = M p, pDp_j = |Dp_j|^2, alpha_j = rr_j / pDp_j
-        if ((rc = meo_mr(c, prec, DP_->data, P_->data, T_->data, s_.kappa, +1, EPI_AXPY_NORM, N, all_done, st, &ps)))
+        if ((rc = meo_mr(c, prec, DP_->data, ring_.p[q], T_->data, s_.kappa, +1, EPI_AXPY_NORM, N, all_done, st, &ps)))
             return rc;
-        HIPCHK(launch_finish_mr(c->partials, ps, ps, N, st, nullptr, FIN_ALPHA, all_done, S));
-        // DDp = M^dag Dp fused with x_j += alpha_j p_j, r_j -= alpha_j DDp_j, rrnew_j = |r_j|^2
+        HIPCHK(launch_finish_mr(c->partials, ps, ps, N, st, nullptr, FIN_ALPHA, all_done, S, q));
+        // DDp = M^dag Dp fused with r_j -= alpha_j DDp_j, rrnew_j = |r_j|^2
         if ((rc = dslash_mr_all(c, prec, T_->data, 1, DP_->data, nullptr, -s_.kappa, -1, EPI_SET, N, all_done,
-                                st, nullptr, nullptr, nullptr, nullptr)))
+                                st, nullptr, nullptr)))
             return rc;
         if ((rc = dslash_mr_all(c, prec, nullptr, 0, T_->data, DP_->data, s_.kappa, -1, EPI_CGUPD, N, all_done,
-                                st, acc_, P_->data, R_->data, &ps)))
+                                st, R_->data, &ps)))
             return rc;
         HIPCHK(launch_finish_mr(c->partials, ps, ps, N, st, nullptr, s_.mixed ? FIN_RRNEW_MIXED2 : FIN_RRNEW,
                                 all_done, S));
         HIPCHK(launch_batch_sync(st, N, s_.mixed ? 1 : 0, c->flags_d, nullptr, S));
-        // p_j = beta_j p_j + r_j
-        HIPCHK(launch_xpay_mr(prec, c->g, P_->data, R_->data, st, all_done, N, S));
+        // p_j = beta_j p_j + r_j, and x_j (or y_j) of a full ring
+        HIPCHK(launch_xpay_mr(prec, c->g, ring_, q, R_->data, acc_, st, all_done, N, S));
     }
     if (s_.mixed)
         if ((rc = enqueue_update())) return rc;
@@ -491,7 +507,7 @@ int BatchCG::enqueue_update() {
     const int *gate = c->flags_d + 2;
     const int N = N_, prec = s_.prec;
     int rc;
-    if (Y_) HIPCHK(launch_fold_mr(c->g, x_, Y_->data, st, 0, N, gate, S));
+    HIPCHK(launch_flush_mr(prec, c->g, ring_, x_, Y_ ? Y_->data : nullptr, st, 0, N, gate, S));
     if ((rc = meo_mr(c, WL_F64, DP64_->data, x_, T64_->data, s_.kappa, +1, EPI_AXPY, N, gate, nullptr, nullptr)))
         return rc;
     if ((rc = meo_mr(c, WL_F64, DDP64_->data, DP64_->data, T64_->data, s_.kappa, -1, EPI_AXPY, N, gate, nullptr,
@@ -499,7 +515,8 @@ int BatchCG::enqueue_update() {
         return rc;
     HIPCHK(launch_residual_update_mr(prec, c->g, b_, DDP64_->data, R_->data, st, 0, N, c->partials, gate, S));
     HIPCHK(launch_finish_mr(c->partials, pplain_, pplain_, N, st, nullptr, FIN_UPDATE, gate, S));
-    HIPCHK(launch_xpay_mr(prec, c->g, P_->data, R_->data, st, gate, N, S));
+    // p_j = beta_j p_j + r_j in slot 0
+    HIPCHK(launch_xpay_mr(prec, c->g, PRing{{P_->data, P_->data}, 2}, 0, R_->data, nullptr, st, gate, N, S));
     HIPCHK(launch_batch_sync(st, N, 0, c->flags_d, gate, S));
     return WL_OK;
 }
@@ -511,7 +528,7 @@ int BatchCG::enqueue_final() {
     CgState *st = c->st_mr;
     const int N = N_;
     int rc;
-    if (Y_) HIPCHK(launch_fold_mr(c->g, x_, Y_->data, st, 1, N, nullptr, S));
+    HIPCHK(launch_flush_mr(s_.prec, c->g, ring_, x_, Y_ ? Y_->data : nullptr, st, 1, N, nullptr, S));
     // In mixed precision an rhs converges only at a reliable update, which has just computed
     // its FP64 true residual for the final x: the recomputation runs only if some rhs ended
     // otherwise (maxiters).  Plain CG always recomputes it.

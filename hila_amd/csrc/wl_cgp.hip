@@ -130,7 +130,7 @@ __device__ void hop_pass(const CgpArgs &P, cx<double> *out, int out_par, const c
         const int k = lane_site_of(P.g, vb, P.nbh);
         double nrm = 0;
         if (k < P.g.vh) nrm = dslash_site<double, SIGN, EPI, LF>(A, k, sst->alpha);
-        if constexpr (EPI == EPI_AXPY_NORM || EPI == EPI_CGUPD) {
+        if constexpr (EPI == EPI_AXPY_NORM || EPI == EPI_CGUPDX) {
             const double bs = block_sum(nrm);
             if (threadIdx.x == 0) P.partials[vb] = bs;
         }
@@ -197,7 +197,7 @@ __device__ bool cg_body(const CgpArgs &P, CgState *sst) {
         finish(P, P.nbh, FIN_ALPHA, sst);
         hop_pass<-1, EPI_SET, LF>(P, P.t, 1, P.Dp, nullptr, -P.kappa, sst);
         WL_SYNC();
-        hop_pass<-1, EPI_CGUPD, LF>(P, nullptr, 0, P.t, P.Dp, P.kappa, sst);
+        hop_pass<-1, EPI_CGUPDX, LF>(P, nullptr, 0, P.t, P.Dp, P.kappa, sst);
         WL_SYNC();
         finish(P, P.nbh, FIN_RRNEW, sst);
         if (sst->done) break;

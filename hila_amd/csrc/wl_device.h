@@ -378,6 +378,10 @@ __device__ __forceinline__ double block_sum(double v) {
     return s;
 }
 
+// Search directions kept by a solve: x += alpha_i p_i of up to kRing iterations is done in one pass
+// (PRing, wl_internal.h).
+constexpr int kRing = 4;
+
 // Device-resident scalars of one CG solve (conjugate_gradient.h:55-57), updated by the last
 // workgroup of each reduction kernel so that no scalar leaves the device inside the loop.
 // `done` stops every gated kernel of the loop while non-zero:
@@ -392,6 +396,9 @@ struct CgState {
                         // rr_i
     double rr_update;   // ||r||^2 at the last reliable update
     double delta2;      // update when ||r||^2 < delta2 * rr_update
+    double alphas[kRing];  // alpha of the iteration whose search direction is in each ring slot
+    int pend;           // slots 0 .. pend - 1 are not yet in x; holds once the solve has stopped or
+                        // paused (done != 0)
     int iter, done, maxiters, nreliable;
     int iter_since;     // iterations since the last reliable update
     int update_every;   // ... or after this many iterations
@@ -416,6 +423,7 @@ struct RedArgs {
     double *partials;   // one slot per workgroup of the reducing kernel
     CgState *st;
     double *out;        // FIN_STORE target
+    int slot = 0;       // FIN_ALPHA: ring slot of the iteration's search direction
 };
 
 __device__ __forceinline__ void fin_apply(int fin, double s, const RedArgs &ra) {
@@ -434,6 +442,8 @@ __device__ __forceinline__ void fin_apply(int fin, double s, const RedArgs &ra) 
     case FIN_ALPHA:
         st->pDp = s;
         st->alpha = st->rr / s;
+        st->alphas[ra.slot] = st->alpha;
+        st->pend = ra.slot + 1;
         break;
     case FIN_RRNEW:
         st->rrnew = s;
@@ -473,6 +483,7 @@ __device__ __forceinline__ void fin_apply(int fin, double s, const RedArgs &ra) 
     case FIN_UPDATE:
         st->true_rr = s;
         st->nreliable += 1;
+        st->pend = 0;
         if (s < st->target_rr) {
             st->rrnew = s;
             st->done = 1;

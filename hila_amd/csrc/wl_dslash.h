@@ -9,6 +9,9 @@
 
 namespace wl {
 
+template <int EPI>
+constexpr bool kUpdates = EPI == EPI_CGUPD || EPI == EPI_CGUPDX;
+
 template <typename R>
 struct DslashArgs {
     cx<R> *__restrict__ out;
@@ -20,8 +23,8 @@ struct DslashArgs {
     Geom g;
     int out_par;
     const int *done;
-    cx<double> *__restrict__ x;   // the solution is accumulated in FP64 at every precision
-    const cx<R> *__restrict__ p;
+    cx<double> *__restrict__ x;   // EPI_CGUPDX: the solution, FP64 at every precision
+    const cx<R> *__restrict__ p;  // EPI_CGUPDX
     cx<R> *__restrict__ r;
     RedArgs red;
     int fin;
@@ -44,6 +47,8 @@ __device__ __forceinline__ double cg_alpha(const DslashArgs<R> &A) {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         A.red.st->pDp = s;
         A.red.st->alpha = alpha;
+        A.red.st->alphas[A.red.slot] = alpha;
+        A.red.st->pend = A.red.slot + 1;
     }
     return alpha;
 }
@@ -79,26 +84,28 @@ __device__ __forceinline__ double dslash_site(const DslashArgs<R> &A, int k, dou
                     if constexpr (EPI == EPI_AXPY_NORM) nrm += (double)norm2(v[s][c]);
                 }
             st_site<R, true>(A.out, S, k, v);
-        } else {  // EPI_CGUPD: x (FP64) += alpha p, r -= alpha DDp in R
+        } else {  // EPI_CGUPD, EPI_CGUPDX: r -= alpha DDp in R; x (FP64) += alpha p
             const R alpha_r = (R)alpha;
-            cx<R> ddp[4][3], pv[4][3], rv[4][3];
+            cx<R> ddp[4][3], rv[4][3];
             ld_site<R, true>(A.xin, S, k, ddp);
             scale_unless_one(ddp, A.b);
-            ld_site<R, true>(A.p, S, k, pv);
             ld_site<R, true>(A.r, S, k, rv);
-            cx<double> xv[4][3];
-            ld_site<double, true>(A.x, S, k, xv);
+            if constexpr (EPI == EPI_CGUPDX) {
+                cx<R> pv[4][3];
+                cx<double> xv[4][3];
+                ld_site<R, true>(A.p, S, k, pv);
+                ld_site<double, true>(A.x, S, k, xv);
+                x_add<R>(xv, alpha, pv);
+                st_site<double, true>(A.x, S, k, xv);
+            }
 #pragma unroll
             for (int s = 0; s < 4; ++s)
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {
-                    const cx<double> pd = {(double)pv[s][c].x, (double)pv[s][c].y};
-                    xv[s][c] = xv[s][c] + alpha * pd;
                     const cx<R> dd = ddp[s][c] + a * acc[s][c];
                     rv[s][c] = rv[s][c] - alpha_r * dd;
                     nrm += (double)norm2(rv[s][c]);
                 }
-            st_site<double, true>(A.x, S, k, xv);
             st_site<R, true>(A.r, S, k, rv);
         }
     }

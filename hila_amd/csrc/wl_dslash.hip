@@ -28,11 +28,11 @@ template <typename R, int SIGN, int EPI, int LF>
 __global__ __launch_bounds__(kBlock) void k_dslash(DslashArgs<R> A) {
     if (A.done && *A.done) return;
     double alpha = 0;
-    if constexpr (EPI == EPI_CGUPD) alpha = cg_alpha(A);
+    if constexpr (kUpdates<EPI>) alpha = cg_alpha(A);
     const int k = lane_site(A.g);
     double nrm = 0;
     if (k < A.g.vh) nrm = dslash_site<R, SIGN, EPI, LF>(A, k, alpha);
-    if constexpr (EPI == EPI_AXPY_NORM || EPI == EPI_CGUPD) reduce_partial(nrm, A.red);
+    if constexpr (EPI == EPI_AXPY_NORM || kUpdates<EPI>) reduce_partial(nrm, A.red);
 }
 
 // ------------------------------------------------------------ small lattices ------------
@@ -62,7 +62,7 @@ template <typename R, int SIGN, int EPI, int LF>
 __global__ __launch_bounds__(256) void k_dslash_dir(DslashArgs<R> A) {
     if (A.done && *A.done) return;
     double alpha = 0;
-    if constexpr (EPI == EPI_CGUPD) alpha = cg_alpha(A);
+    if constexpr (EPI == EPI_CGUPDX) alpha = cg_alpha(A);
     __shared__ cx<R> part[4][12][64];  // [direction][component][site]
     const int w = (int)(threadIdx.x >> 6), l = (int)(threadIdx.x & 63);
     const int k = xcd_tile(blockIdx.x, gridDim.x) * 64 + l;
@@ -80,9 +80,9 @@ __global__ __launch_bounds__(256) void k_dslash_dir(DslashArgs<R> A) {
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
             if constexpr (EPI != EPI_SET) xi[c] = ldc<true>(A.xin + e[c]);
-            if constexpr (EPI == EPI_CGUPD) {
-                pv[c] = ldc<true>(A.p + e[c]);
+            if constexpr (EPI == EPI_CGUPDX) {
                 rv[c] = ldc<true>(A.r + e[c]);
+                pv[c] = ldc<true>(A.p + e[c]);
                 xv[c] = ldc<true>(A.x + ex[c]);
             }
         }
@@ -123,7 +123,7 @@ __global__ __launch_bounds__(256) void k_dslash_dir(DslashArgs<R> A) {
                 if constexpr (EPI == EPI_AXPY_NORM) nrm += (double)norm2(v);
                 stc<true>(A.out + e[c], v);
             }
-        } else {  // EPI_CGUPD: x (FP64) += alpha p, r -= alpha DDp
+        } else {  // EPI_CGUPDX: x (FP64) += alpha p, r -= alpha DDp
             const R alpha_r = (R)alpha;
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
@@ -139,7 +139,7 @@ __global__ __launch_bounds__(256) void k_dslash_dir(DslashArgs<R> A) {
             }
         }
     }
-    if constexpr (EPI == EPI_AXPY_NORM || EPI == EPI_CGUPD) reduce_partial(nrm, A.red);
+    if constexpr (EPI == EPI_AXPY_NORM || EPI == EPI_CGUPDX) reduce_partial(nrm, A.red);
 }
 
 // Default workgroup size, from measurements on MI355X (256 CUs): 256 lanes from 2^19 sites
@@ -177,19 +177,23 @@ static hipError_t launch_t(const Geom &g, const DslashLaunch &L, hipStream_t s) 
     A.fold_n = L.fold_n;
     A.fold_it = L.fold_it;
     const int nb = hop_blocks(g);
-    if (g.dir) {
-        if (L.lf == 6)
+    // solves on small lattices keep no ring of search directions, the others do
+    if ((EPI == EPI_CGUPDX && !g.dir) || (EPI == EPI_CGUPD && g.dir)) return hipErrorInvalidValue;
+    if constexpr (EPI != EPI_CGUPD) {
+        if (g.dir && L.lf == 6)
             hipLaunchKernelGGL((k_dslash_dir<R, SIGN, EPI, 6>), dim3(nb), dim3(256), 0, s, A);
-        else
+        else if (g.dir)
             hipLaunchKernelGGL((k_dslash_dir<R, SIGN, EPI, 9>), dim3(nb), dim3(256), 0, s, A);
-    } else if (L.lf == 6) {
-        hipLaunchKernelGGL((k_dslash<R, SIGN, EPI, 6>), dim3(nb), dim3(g.blk), g.lds, s, A);
-    } else {
-        hipLaunchKernelGGL((k_dslash<R, SIGN, EPI, 9>), dim3(nb), dim3(g.blk), g.lds, s, A);
+    }
+    if constexpr (EPI != EPI_CGUPDX) {
+        if (!g.dir && L.lf == 6)
+            hipLaunchKernelGGL((k_dslash<R, SIGN, EPI, 6>), dim3(nb), dim3(g.blk), g.lds, s, A);
+        else if (!g.dir)
+            hipLaunchKernelGGL((k_dslash<R, SIGN, EPI, 9>), dim3(nb), dim3(g.blk), g.lds, s, A);
     }
     hipError_t e = hipGetLastError();
     // FIN_NONE: the partials are left for the next kernel (launch-folded CG)
-    if (e != hipSuccess || (EPI != EPI_AXPY_NORM && EPI != EPI_CGUPD) || L.fin == FIN_NONE) return e;
+    if (e != hipSuccess || (EPI != EPI_AXPY_NORM && !kUpdates<EPI>) || L.fin == FIN_NONE) return e;
     return launch_finish(L.red, nb, L.fin, L.done, s);
 }
 
@@ -203,19 +207,19 @@ static hipError_t launch_epi(const Geom &g, const DslashLaunch &L, hipStream_t s
     }
 }
 
+// The CG's update pass is M^dag's second half (sign -1).
+template <typename R>
+static hipError_t launch_prec(const Geom &g, const DslashLaunch &L, hipStream_t s) {
+    if (L.epi == EPI_CGUPD || L.epi == EPI_CGUPDX) {
+        if (L.sign > 0) return hipErrorInvalidValue;
+        return L.epi == EPI_CGUPD ? launch_t<R, -1, EPI_CGUPD>(g, L, s) : launch_t<R, -1, EPI_CGUPDX>(g, L, s);
+    }
+    return L.sign > 0 ? launch_epi<R, 1>(g, L, s) : launch_epi<R, -1>(g, L, s);
+}
+
 hipError_t launch_dslash(int prec, const Geom &g, const DslashLaunch &L, hipStream_t s) {
-    if (prec == WL_F64) {
-        if (L.epi == EPI_CGUPD)
-            return L.sign > 0 ? launch_t<double, 1, EPI_CGUPD>(g, L, s)
-                              : launch_t<double, -1, EPI_CGUPD>(g, L, s);
-        return L.sign > 0 ? launch_epi<double, 1>(g, L, s) : launch_epi<double, -1>(g, L, s);
-    }
-    if (prec == WL_F32) {
-        if (L.epi == EPI_CGUPD)
-            return L.sign > 0 ? launch_t<float, 1, EPI_CGUPD>(g, L, s)
-                              : launch_t<float, -1, EPI_CGUPD>(g, L, s);
-        return L.sign > 0 ? launch_epi<float, 1>(g, L, s) : launch_epi<float, -1>(g, L, s);
-    }
+    if (prec == WL_F64) return launch_prec<double>(g, L, s);
+    if (prec == WL_F32) return launch_prec<float>(g, L, s);
     return hipErrorInvalidValue;
 }
 

@@ -123,8 +123,8 @@ int rhs_per_launch(const wl_ctx *c, int nr, int N);
 // out = a H_sign in (+ epilogue) for N right-hand sides; per-rhs partial sums land in
 // c->partials rows, *pstride_out apart.
 int dslash_mr_all(wl_ctx *c, int prec, void *out, int out_par, const void *in, const void *xin,
-                  double a, int sign, int epi, int N, const int *all_done, CgState *st, void *x,
-                  const void *p, void *r, int *pstride_out);
+                  double a, int sign, int epi, int N, const int *all_done, CgState *st, void *r,
+                  int *pstride_out);
 // M_s for N right-hand sides (even fields) through the odd work field t
 int meo_mr(wl_ctx *c, int prec, void *out, const void *in, void *t, double kappa, int sign,
            int epi2, int N, const int *all_done, CgState *st, int *pstride_out);

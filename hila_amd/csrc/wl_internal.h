@@ -31,7 +31,22 @@ enum Epi : int {
     EPI_SET = 0,        // out = a H in                           (Dirac_Wilson_hop_set)
     EPI_AXPY = 1,       // out = xin + a H in                     (second half of M)
     EPI_AXPY_NORM = 2,  // out = xin + a H in, reduce ||out||^2   (M p with pDp fused)
-    EPI_CGUPD = 3,      // DDp = xin + a H in; x += alpha p; r -= alpha DDp; reduce ||r||^2
+    EPI_CGUPD = 3,      // r -= alpha (xin + a H in), i.e. alpha DDp; reduce ||r||^2
+    EPI_CGUPDX = 4,     // and x += alpha p (where the search directions have no ring)
+};
+
+// Search directions of a solve: iteration i's p is in slot i % n, and the pass that writes the
+// next p into slot 0 first adds all n to the solution, x += sum alpha_i p_i in order: the same
+// sums, but x is read and written once for n iterations, and p not at all by the pass that
+// updates r.  Per site and iteration FP64 moves 288 bytes for x and p with two slots instead of
+// 576, FP32 with an FP64 x 168 with four instead of 480, FP16 with an FP32 one 87 instead of 244.
+// Slots past the first are in work fields that idle between the true residuals.  n = 1: no ring, the
+// pass that updates r updates x (EPI_CGUPDX).  That is the faster way where the lattice sits in
+// the caches and a launch is latency: 8^4 in FP64, the ring made p = beta p + r 3.6 -> 4.6 us a
+// launch and left the update pass at 6.2.
+struct PRing {
+    void *p[kRing];
+    int n;
 };
 
 struct DslashLaunch {
@@ -46,10 +61,9 @@ struct DslashLaunch {
     int sign;      // +1 apply, -1 dagger
     int epi;
     const int *done;  // skip the launch body when *done != 0 (CG loop); may be null
-    // EPI_CGUPD operands (FP64 even fields)
-    void *x;
+    void *r;               // EPI_CGUPD
+    void *x;               // EPI_CGUPDX: FP64, and p
     const void *p;
-    void *r;
     RedArgs red;
     int fin;               // applied by a finish kernel after a norm epilogue; FIN_NONE: none
     // EPI_CGUPD of the launch-folded CG: alpha from fold_n partials (DslashArgs); null: none
@@ -92,13 +106,18 @@ hipError_t launch_norm2(int prec, const Geom &g, const void *f, int N, int j, co
 // r = b - DDp; p = r; reduce ||r||^2 -> FIN_RR   (conjugate_gradient.h:67-72)
 hipError_t launch_cg_init(const Geom &g, const void *b, const void *DDp, void *r, void *p,
                           const RedArgs &ra, hipStream_t s);
-// p = beta p + r, beta from the CG state (conjugate_gradient.h:93-94); skipped when done != 0
-hipError_t launch_cg_xpay(int prec, const Geom &g, void *p, const void *r, const CgState *st,
-                          hipStream_t s);
-// the same in FP64 for iteration `it` of the launch-folded CG, with the finish of the n partials
-// of ||r||^2 at `parts` folded in (convergence test, beta, state; k_cg_xpay_fold)
-hipError_t launch_cg_xpay_fold(const Geom &g, void *p, const void *r, CgState *st, const double *parts, int n,
-                               int it, hipStream_t s);
+// next p = beta p + r from ring slot q, beta from the CG state (conjugate_gradient.h:93-94), with
+// the x update of a full ring (x FP64); skipped when done != 0
+hipError_t launch_cg_xpay(int prec, const Geom &g, const PRing &ring, int q, const void *r, void *x,
+                          const CgState *st, hipStream_t s);
+// p = beta p + r in slot 0 (restart after a reliable update); skipped when done != 0
+hipError_t launch_cg_restart(int prec, const Geom &g, void *p, const void *r, const CgState *st, hipStream_t s);
+// launch_cg_xpay in FP64 for iteration `it` of the launch-folded CG, with the finish of the n
+// partials of ||r||^2 at `parts` folded in (convergence test, beta, state; k_cg_xpay_fold)
+hipError_t launch_cg_xpay_fold(const Geom &g, const PRing &ring, const void *r, void *x, CgState *st,
+                               const double *parts, int n, int it, hipStream_t s);
+// x += alpha p of the slots a stopped or paused solve has not added; its last p to slot 0
+hipError_t launch_cg_flush(int prec, const Geom &g, const PRing &ring, void *x, const CgState *st, hipStream_t s);
 // reliable update: r_lo = b - DDp (FP64 in, inner precision out), ||.||^2 -> FIN_UPDATE
 hipError_t launch_residual_update(int prec, const Geom &g, const void *b, const void *DDp,
                                   void *r_lo, const RedArgs &ra, hipStream_t s);
@@ -130,9 +149,7 @@ struct MrLaunch {
     bool pipe;                // software-pipelined hops where the registers allow
     const int *all_done;      // may be null
     CgState *st;              // per-rhs states (skip finished rhs, alpha); may be null
-    void *x;                  // EPI_CGUPD accumulator: FP64 x (FP64 arithmetic) or FP32 y
-    const void *p;
-    void *r;
+    void *r;                  // EPI_CGUPD
     double *partials;
 };
 // Tiles of the LDS-tiled FP16 hopping kernel (wl_tile.h): ty x tz rows (a row: all x) of one time
@@ -192,7 +209,7 @@ hipError_t launch_dslash_tile(const Geom &g, const TileGeom &tg, const MrLaunch 
 hipError_t launch_dslash_mr(int prec, const Geom &g, const MrLaunch &L, hipStream_t s);
 int mr_segments(const Geom &g);
 hipError_t launch_finish_mr(double *partials, int pstride, int n, int N, CgState *st,
-                            double *out, int fin, const int *all_done, hipStream_t s);
+                            double *out, int fin, const int *all_done, hipStream_t s, int slot = 0);
 // BLAS-1 kernels over N right-hand sides: per-rhs partials at partials[rhs * nblocks(g) + b]
 hipError_t launch_norm2_mr(int prec, const Geom &g, const void *f, int N, double *partials,
                            hipStream_t s);
@@ -201,8 +218,13 @@ hipError_t launch_cg_init_mr(const Geom &g, const void *b, const void *ddp, void
 hipError_t launch_residual_update_mr(int prec, const Geom &g, const void *b, const void *ddp,
                                      void *r, const CgState *st, int first, int N,
                                      double *partials, const int *gate, hipStream_t s);
-hipError_t launch_xpay_mr(int prec, const Geom &g, void *p, const void *r, const CgState *st,
-                          const int *all_done, int N, hipStream_t s);
+// launch_cg_xpay for the running rhs; acc: FP64 x (FP64 arithmetic) or the FP32 inner solution
+hipError_t launch_xpay_mr(int prec, const Geom &g, const PRing &ring, int q, const void *r, void *acc,
+                          const CgState *st, const int *all_done, int N, hipStream_t s);
+// launch_cg_flush for every rhs (all) or those taking a reliable update; with an FP32 inner
+// solution y, x += y and y = 0 too
+hipError_t launch_flush_mr(int prec, const Geom &g, const PRing &ring, void *x, void *y, const CgState *st, int all,
+                           int N, const int *gate, hipStream_t s);
 // flags[0] all finished, flags[1] update pending, flags[2] no update pending; gate: skip if set
 hipError_t launch_batch_sync(CgState *st, int N, int mixed, int *flags, const int *gate,
                              hipStream_t s);

@@ -5,6 +5,7 @@
 // (conjugate_gradient.h:75-95) with its own alpha, beta and convergence flag, and all share
 // every operator application.  Per-rhs partial sums are reduced in a fixed order.
 
+#include "wl_blas.h"
 #include "wl_hop.h"
 #include "wl_internal.h"
 #include "wl_store.h"
@@ -85,26 +86,65 @@ __global__ __launch_bounds__(kBlock) void k_residual_update_mr(
     if (threadIdx.x == 0) partials[(size_t)j * gridDim.x + blockIdx.x] = s;
 }
 
-// p = beta_j p + r for the rhs still running (done == 0)
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_xpay_mr(typename St<T>::E *__restrict__ p,
-                                                    const typename St<T>::E *__restrict__ r,
-                                                    const CgState *st, const int *all_done,
-                                                    int vh, int S) {
+// Next p = beta_j p + r of the rhs still running (done == 0), from ring slot q to slot q + 1; X
+// (the ring is full): into slot 0, after x += alpha p of all slots, q the last of them (x: the FP64
+// solution in FP64 arithmetic, else the FP32 inner one).
+template <typename T, bool X>
+__global__ __launch_bounds__(kBlock) void k_xpay_mr(RingArgs<T> ring, int q, const typename St<T>::E *__restrict__ r,
+                                                    cx<typename St<T>::R> *__restrict__ x, const CgState *st,
+                                                    const int *all_done, int vh, int S) {
     using R = typename St<T>::R;
     if (all_done && *all_done) return;
     const int k = blockIdx.x * kBlock + threadIdx.x, j = blockIdx.y;
     if (k >= vh || st[j].done) return;
-    const R beta = (R)st[j].beta;
     const size_t off = (size_t)j * St<T>::planes * S;
-    cx<R> pv[4][3], rv[4][3];
-    ld_site<T>(p + off, S, k, pv);
-    ld_site<T>(r + off, S, k, rv);
+    cx<R> pv[4][3];
+    if constexpr (X)
+        site_ring<T, R>(x + (size_t)j * 12 * S, ring, st[j].alphas, q + 1, off, S, k, pv);
+    else
+        ld_site<T>(ring.p[q] + off, S, k, pv);
+    site_xpay<T>(ring.p[X ? 0 : q + 1] + off, pv, r + off, (R)st[j].beta, S, k);
+}
+
+// The solution of the rhs that take a reliable update (done 3 or 4), or of every rhs that has
+// stopped with all != 0: x += alpha p of the pending ring slots, and the last p to slot 0.  With
+// an inner solution y (Y), into y first, and then x += y, y = 0.  Skipped when *gate != 0.
+template <typename T, bool Y>
+__global__ __launch_bounds__(kBlock) void k_flush_mr(RingArgs<T> ring, cx<double> *__restrict__ x,
+                                                     cx<float> *__restrict__ y, const CgState *st, int all, int vh,
+                                                     int S, const int *gate) {
+    using R = typename St<T>::R;
+    if (gate && *gate) return;
+    const int k = blockIdx.x * kBlock + threadIdx.x, j = blockIdx.y;
+    const int done = st[j].done;
+    if (k >= vh || !(all || done == 3 || done == 4)) return;
+    const int n = done ? st[j].pend : 0;
+    const size_t off = (size_t)j * St<T>::planes * S, xoff = (size_t)j * 12 * S;
+    cx<R> pv[4][3];
+    if constexpr (Y) {
+        cx<R> yv[4][3];
+        cx<double> xv[4][3];
+        ld_site<R, true>((cx<R> *)y + xoff, S, k, yv);
+        ld_site<double, true>(x + xoff, S, k, xv);
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+        for (int m = 0; m < kRing; ++m)
+            if (m < n) {
+                ld_site<T>(ring.p[m] + off, S, k, pv);
+                x_add<R>(yv, (R)st[j].alphas[m], pv);
+            }
 #pragma unroll
-        for (int c = 0; c < 3; ++c) pv[a][c] = beta * pv[a][c] + rv[a][c];
-    st_site<T>(p + off, S, k, pv);
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                xv[s][c] = xv[s][c] + cx<double>{(double)yv[s][c].x, (double)yv[s][c].y};
+                yv[s][c] = {R(0), R(0)};
+            }
+        st_site<double, true>(x + xoff, S, k, xv);
+        st_site<R, true>((cx<R> *)y + xoff, S, k, yv);
+    } else if (n) {
+        site_ring<T, double>(x + xoff, ring, st[j].alphas, n, off, S, k, pv);
+    }
+    if (n > 1) st_site<T>(ring.p[0] + off, S, k, pv);
 }
 
 // Fold the inner solution into the FP64 one: x_j += y_j, y_j = 0, for the rhs that take a
@@ -149,7 +189,7 @@ __global__ __launch_bounds__(kBlock) void k_zero_rhs(cx<double> *__restrict__ x,
 // rhs that asked for an update for FIN_UPDATE, every rhs otherwise).
 __global__ __launch_bounds__(kBlock) void k_finish_mr(double *partials, int pstride, int n,
                                                       CgState *st, double *out, int fin,
-                                                      const int *all_done) {
+                                                      const int *all_done, int slot) {
     if (all_done && *all_done) return;
     const int j = blockIdx.x;
     const int d = st ? st[j].done : 0;
@@ -166,6 +206,7 @@ __global__ __launch_bounds__(kBlock) void k_finish_mr(double *partials, int pstr
         ra.partials = partials;
         ra.st = st ? st + j : nullptr;
         ra.out = out ? out + j : nullptr;
+        ra.slot = slot;
         fin_apply(fin == FIN_UPDATE_FIRST ? FIN_UPDATE : fin, s, ra);
     }
 }
@@ -228,9 +269,9 @@ hipError_t launch_dslash_mr(int prec, const Geom &g, const MrLaunch &L, hipStrea
 }
 
 hipError_t launch_finish_mr(double *partials, int pstride, int n, int N, CgState *st,
-                            double *out, int fin, const int *all_done, hipStream_t s) {
+                            double *out, int fin, const int *all_done, hipStream_t s, int slot) {
     hipLaunchKernelGGL(k_finish_mr, dim3(N), dim3(kBlock), 0, s, partials, pstride, n, st, out,
-                       fin, all_done);
+                       fin, all_done, slot);
     return hipGetLastError();
 }
 
@@ -278,18 +319,54 @@ hipError_t launch_residual_update_mr(int prec, const Geom &g, const void *b, con
     return hipGetLastError();
 }
 
-hipError_t launch_xpay_mr(int prec, const Geom &g, void *p, const void *r, const CgState *st,
-                          const int *all_done, int N, hipStream_t s) {
+template <typename T>
+static RingArgs<T> ring_args(const PRing &ring) {
+    RingArgs<T> a;
+    for (int m = 0; m < kRing; ++m) a.p[m] = (typename St<T>::E *)(m < ring.n ? ring.p[m] : nullptr);
+    return a;
+}
+
+template <typename T>
+static void xpay_mr_t(const Geom &g, const PRing &ring, int q, const void *r, void *acc, const CgState *st,
+                      const int *all_done, int N, hipStream_t s) {
     const dim3 grid(nblocks(g), N);
-    if (prec == WL_F64)
-        hipLaunchKernelGGL(k_xpay_mr<double>, grid, dim3(kBlock), 0, s, (cx<double> *)p,
-                           (const cx<double> *)r, st, all_done, g.vh, g.stride);
-    else if (prec == WL_F32)
-        hipLaunchKernelGGL(k_xpay_mr<float>, grid, dim3(kBlock), 0, s, (cx<float> *)p,
-                           (const cx<float> *)r, st, all_done, g.vh, g.stride);
-    else if (prec == WL_F16)
-        hipLaunchKernelGGL(k_xpay_mr<f16s>, grid, dim3(kBlock), 0, s, (h2 *)p, (const h2 *)r, st, all_done,
+    const auto *R = (const typename St<T>::E *)r;
+    auto *X = (cx<typename St<T>::R> *)acc;
+    if (q == ring.n - 1)
+        hipLaunchKernelGGL((k_xpay_mr<T, true>), grid, dim3(kBlock), 0, s, ring_args<T>(ring), q, R, X, st, all_done,
                            g.vh, g.stride);
+    else
+        hipLaunchKernelGGL((k_xpay_mr<T, false>), grid, dim3(kBlock), 0, s, ring_args<T>(ring), q, R, X, st, all_done,
+                           g.vh, g.stride);
+}
+
+hipError_t launch_xpay_mr(int prec, const Geom &g, const PRing &ring, int q, const void *r, void *acc,
+                          const CgState *st, const int *all_done, int N, hipStream_t s) {
+    if (prec == WL_F64)
+        xpay_mr_t<double>(g, ring, q, r, acc, st, all_done, N, s);
+    else if (prec == WL_F32)
+        xpay_mr_t<float>(g, ring, q, r, acc, st, all_done, N, s);
+    else if (prec == WL_F16)
+        xpay_mr_t<f16s>(g, ring, q, r, acc, st, all_done, N, s);
+    else
+        return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+hipError_t launch_flush_mr(int prec, const Geom &g, const PRing &ring, void *x, void *y, const CgState *st, int all,
+                           int N, const int *gate, hipStream_t s) {
+    const dim3 grid(nblocks(g), N);
+    cx<double> *X = (cx<double> *)x;
+    cx<float> *Yv = (cx<float> *)y;
+    if (prec == WL_F64 && !y)
+        hipLaunchKernelGGL((k_flush_mr<double, false>), grid, dim3(kBlock), 0, s, ring_args<double>(ring), X, Yv, st,
+                           all, g.vh, g.stride, gate);
+    else if (prec == WL_F32 && y)
+        hipLaunchKernelGGL((k_flush_mr<float, true>), grid, dim3(kBlock), 0, s, ring_args<float>(ring), X, Yv, st, all,
+                           g.vh, g.stride, gate);
+    else if (prec == WL_F16 && y)
+        hipLaunchKernelGGL((k_flush_mr<f16s, true>), grid, dim3(kBlock), 0, s, ring_args<f16s>(ring), X, Yv, st, all,
+                           g.vh, g.stride, gate);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();

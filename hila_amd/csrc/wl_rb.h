@@ -44,8 +44,6 @@ struct RbArgs {
     int j0, jend, C;           // right-hand sides [j0, jend) in chunks of NR; C chunks
     const int *all_done;       // skip the launch when set (batched CG loop); may be null
     CgState *st;               // per-rhs CG states (skip finished rhs, alpha); may be null
-    cx<R> *__restrict__ x;     // solution accumulator: x itself (FP64) or the inner y (FP32)
-    const E *__restrict__ p;
     E *__restrict__ r;
     double *partials;
     int pstride;               // partial sums: partials[rhs * pstride + segment]
@@ -260,21 +258,17 @@ __device__ __forceinline__ void rb_epilogue(const RbArgs<T> &A, cx<typename St<T
 #pragma unroll
                     for (int c = 0; c < 3; ++c) nrm[r] += (double)norm2(v[s][c]);
             }
-        } else {  // EPI_CGUPD: x += alpha p (x: FP64 solution or FP32 inner y), r -= alpha DDp
+        } else {  // EPI_CGUPD: r -= alpha DDp
             const double alpha = A.st[jf + r].alpha;
             const R alpha_r = (R)alpha;
-            cx<R> ddp[4][3], pv[4][3], rv[4][3];
+            cx<R> ddp[4][3], rv[4][3];
             ld_site<T, true>(A.xin + eb, S, k, ddp);
             scale_unless_one(ddp, A.b);
-            ld_site<T, true>(A.p + eb, S, k, pv);
             ld_site<T, true>(A.r + eb, S, k, rv);
-            const size_t xb = (size_t)(jf + r) * 12 * S;
 #pragma unroll
             for (int s = 0; s < 4; ++s)
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {
-                    const size_t e = xb + comp_elem<double>(s * 3 + c, S, k);
-                    stc<true>(A.x + e, ldc<true>(A.x + e) + alpha_r * pv[s][c]);
                     const cx<R> dd = ddp[s][c] + a * acc[r][s][c];
                     rv[s][c] = rv[s][c] - alpha_r * dd;
                 }
@@ -492,8 +486,6 @@ inline hipError_t rb_launch(const Geom &g, const MrLaunch &L, hipStream_t s) {
     A.C = (L.NB + NR - 1) / NR;
     A.all_done = L.all_done;
     A.st = L.st;
-    A.x = (cx<R> *)L.x;
-    A.p = (const E *)L.p;
     A.r = (E *)L.r;
     A.partials = L.partials;
     A.pstride = mr_segments(g);
@@ -536,8 +528,6 @@ inline hipError_t rb_launch_lds(const Geom &g, const MrLaunch &L, hipStream_t s)
     A.C = (L.NB + NR - 1) / NR;
     A.all_done = L.all_done;
     A.st = L.st;
-    A.x = (cx<R> *)L.x;
-    A.p = (const E *)L.p;
     A.r = (E *)L.r;
     A.partials = L.partials;
     A.pstride = mr_segments(g);

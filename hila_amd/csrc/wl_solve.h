@@ -90,6 +90,7 @@ class BatchCG {
     wl_field *DP64_ = nullptr, *DDP64_ = nullptr, *T64_ = nullptr;
     wl_field *Y_ = nullptr;  // FP32 inner solution (FP32 / FP16 inner precision), folded into x
     void *acc_ = nullptr;    // what x += alpha p accumulates into: Y_ or x itself (FP64)
+    PRing ring_{};           // search directions: P_, and where there is room the FP64 work fields
     int pplain_ = 0;
     int chunks_ = 0;     // chunks enqueued
     int cap_chunks_ = 0;

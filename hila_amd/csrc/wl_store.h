@@ -268,6 +268,15 @@ __device__ __forceinline__ void st_site(typename St<T>::E *base, int S, int k,
     }
 }
 
+// x += alpha p for a spinor p in arithmetic R, in x's arithmetic A
+template <typename R, typename A>
+__device__ __forceinline__ void x_add(cx<A> (&x)[4][3], A alpha, const cx<R> (&p)[4][3]) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) x[s][c] = x[s][c] + alpha * cx<A>{(A)p[s][c].x, (A)p[s][c].y};
+}
+
 // ------------------------------------ packed FP16 hop arithmetic, FP32 accumulation ------
 // The FP16 hop keeps links and spinors packed as stored: the spin projection is one
 // v_pk_add_f16 per complex number and operand form (one FP16 rounding of each half, the same

@@ -179,16 +179,12 @@ __device__ __forceinline__ double tile_epilogue(const RbArgs<f16s> &A, cx<float>
     } else {
         const double alpha = A.st[j].alpha;
         const float alpha_r = (float)alpha;
-        cx<float> ddp[4][3], pv[4][3];
+        cx<float> ddp[4][3];
         raw_widen(ex, ddp);
         scale_unless_one(ddp, A.b);
         raw_widen(er, v);
-        ld_site<f16s, true>(A.p + eb, S, k, pv);
-        const size_t xb = (size_t)j * 12 * S;
 #pragma unroll
         for (int c = 0; c < 12; ++c) {
-            const size_t e = xb + comp_elem<double>(c, S, k);
-            stc<true>(A.x + e, ldc<true>(A.x + e) + alpha_r * pv[c / 3][c % 3]);
             const cx<float> dd = ddp[c / 3][c % 3] + a * acc[c / 3][c % 3];
             v[c / 3][c % 3] = v[c / 3][c % 3] - alpha_r * dd;
         }
@@ -332,8 +328,6 @@ inline hipError_t tile_launch(const Geom &g, const TileGeom &tg, const MrLaunch 
     A.C = (L.NB + L.NR - 1) / L.NR;
     A.all_done = L.all_done;
     A.st = L.st;
-    A.x = (cx<float> *)L.x;
-    A.p = (const h2 *)L.p;
     A.r = (h2 *)L.r;
     A.partials = L.partials;
     A.pstride = tile_slots(G);
