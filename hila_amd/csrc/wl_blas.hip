@@ -326,9 +326,7 @@ __global__ __launch_bounds__(kBlock) void k_convert(const typename St<Ti>::E *__
 // Sum the n partials in workgroup order and apply `fin` (skipped once the CG has finished).
 __global__ __launch_bounds__(kBlock) void k_finish(RedArgs ra, int n, int fin, const int *done) {
     if (done && *done) return;
-    double s = 0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) s += ra.partials[i];
-    s = block_sum(s);
+    const double s = block_sum(strided_sum(ra.partials, n, threadIdx.x));
     if (threadIdx.x == 0) fin_apply(fin, s, ra);
 }
 

@@ -198,9 +198,7 @@ __global__ __launch_bounds__(kBlock) void k_finish_mr(double *partials, int pstr
     if (fin == FIN_UPDATE) apply = d == 3 || d == 4;
     if (fin == FIN_UPDATE_FIRST) apply = d != 1;  // rhs with b = 0 are finished already
     if (!apply) return;
-    double s = 0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) s += partials[(size_t)j * pstride + i];
-    s = block_sum(s);
+    const double s = block_sum(strided_sum(partials + (size_t)j * pstride, n, threadIdx.x));
     if (threadIdx.x == 0) {
         RedArgs ra;
         ra.partials = partials;
