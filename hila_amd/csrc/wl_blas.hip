@@ -211,41 +211,16 @@ __global__ __launch_bounds__(kBlock) void k_cg_flush(RingArgs<R> ring, cx<double
     if (n > 1) st_site<R>(ring.p[0], S, k, pv);
 }
 
-// p = beta p + r of the launch-folded CG iteration `it` (0-based), with the finish kernel's
-// FIN_RRNEW folded in (conjugate_gradient.h:87-95): every workgroup adds the n partials of
-// ||r||^2 in the finish kernel's order, takes the same convergence decision and beta =
-// rrnew / rr_it, and updates p unless the solve has ended; workgroup 0 records the state
-// (rrnew, iter, done; beta and rr, with rr_(it+1) in slot (it + 1) & 1, unless converged).
-// The done flag is read once per workgroup: workgroup 0 may set it meanwhile, and p is not
-// needed once it is set (the solution then gets the pending slots from launch_cg_flush).  Slots
-// and X as in k_cg_xpay.
+// Next p = beta p + r at the end of iteration `it` of the launch-folded CG, with the finish of that
+// iteration folded in (fold_rrnew); p is not needed once the solve has ended (the solution then
+// gets the pending slots from launch_cg_flush).  Slots and X as in k_cg_xpay.
 template <bool X>
 __global__ __launch_bounds__(kBlock) void k_cg_xpay_fold(const cx<double> *from, cx<double> *to,
                                                          const cx<double> *__restrict__ r, RingArgs<double> ring,
                                                          int nring, cx<double> *__restrict__ x, CgState *st,
                                                          const double *parts, int n, int it, int vh, int S) {
-    __shared__ int ended;
-    if (threadIdx.x == 0) ended = st->done;
-    __syncthreads();
-    if (ended) return;  // workgroup-uniform
-    const double s = finish_order_sum(parts, n);
-    const double rr = st->rrb[it & 1];
-    const int iter = it + 1;
-    const bool conv = s < st->target_rr;
-    const double beta = s / rr;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        st->rrnew = s;
-        st->iter = iter;
-        if (conv) {
-            st->done = 1;
-        } else {
-            st->beta = beta;
-            st->rr = s;
-            st->rrb[(it + 1) & 1] = s;
-            if (iter >= st->maxiters) st->done = 2;
-        }
-    }
-    if (conv || iter >= st->maxiters) return;
+    double beta;
+    if (!fold_rrnew(st, parts, n, it, beta)) return;
     const int k = blockIdx.x * kBlock + threadIdx.x;
     if (k >= vh) return;
     cx<double> pv[4][3];

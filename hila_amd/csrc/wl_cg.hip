@@ -56,7 +56,8 @@ class Pace {
 // the finish of alpha, M^dag Dp fused with the x, r update and ||r||^2 partials, the finish of
 // rrnew (convergence, beta) and p = beta p + r: seven launches.  Folded (cg_fold), the alpha
 // finish moves into the update pass and the rrnew finish into p = beta p + r: five launches,
-// the same sums in the same order, so the same bits.
+// the same sums in the same order, so the same bits.  With the small-lattice kernel (g.dir) the
+// latter move on into the next iteration's first hop: four launches (k_dslash_dir_xpay).
 int cg_f64(wl_ctx *c, const CgWork &w, void *x, size_t x_bytes, const void *b, double kappa, double accuracy,
            int maxiters, wl_cg_stats *stats) {
     const auto t0 = std::chrono::steady_clock::now();
@@ -67,6 +68,8 @@ int cg_f64(wl_ctx *c, const CgWork &w, void *x, size_t x_bytes, const void *b, d
     const RedArgs ra = red_args(w);
     const int *done = &w.st->done;
     const bool fold = cg_fold(c, w);
+    const bool merged = fold && c->g.dir;  // p then moves between p and DDp
+    void *ps = p;
     const int nhop = hop_blocks(c->g);
     double *parts2 = w.partials + nhop;  // folded: partials of the update pass
 
@@ -107,10 +110,32 @@ int cg_f64(wl_ctx *c, const CgWork &w, void *x, size_t x_bytes, const void *b, d
         for (int it = 0; it < n; ++it) {
             RedArgs rs = ra;
             rs.slot = (enqueued + it) % ring.n;
-            void *ps = ring.p[rs.slot];
-            // Dp = M p, pDp = |Dp|^2, alpha = rr / pDp (folded: alpha in the update pass)
-            if ((rc = meo_one(c, rs, WL_F64, Dp, ps, t, kappa, +1, EPI_AXPY_NORM, done, fold ? FIN_NONE : FIN_ALPHA)))
-                return rc;
+            const int fin = fold ? FIN_NONE : FIN_ALPHA;
+            if (merged && it > 0) {
+                // the end of the iteration before, p = beta p + r and t = -kappa H_oe p in one launch
+                DslashLaunch L{};
+                L.out = t;
+                L.in = ps;
+                L.gauge = gauge_for(c, WL_F64);
+                L.lf = link_format(c, WL_F64);
+                if (!L.gauge) return fail(WL_E_STATE, "FP64 links not prepared");
+                L.a = -kappa;
+                L.out_par = 1;
+                L.sign = 1;
+                L.epi = EPI_SET;
+                L.r = r;
+                L.red = rs;
+                L.fold_parts = parts2;
+                L.fold_n = nhop;
+                L.fold_it = enqueued + it - 1;
+                ps = ps == p ? DDp : p;
+                HIPCHK(launch_dslash_xpay(c->g, L, ps, c->stream));
+                if ((rc = dslash_one(c, rs, WL_F64, Dp, 0, t, ps, kappa, +1, EPI_AXPY_NORM, done, fin))) return rc;
+            } else {
+                if (!merged) ps = ring.p[rs.slot];
+                // Dp = M p, pDp = |Dp|^2, alpha = rr / pDp (folded: alpha in the update pass)
+                if ((rc = meo_one(c, rs, WL_F64, Dp, ps, t, kappa, +1, EPI_AXPY_NORM, done, fin))) return rc;
+            }
             // DDp = M^dag Dp fused with r -= alpha DDp, rrnew = |r|^2, test, beta
             if ((rc = dslash_one(c, ra, WL_F64, t, 1, Dp, nullptr, -kappa, -1, EPI_SET, done, FIN_NONE)))
                 return rc;
@@ -128,7 +153,7 @@ int cg_f64(wl_ctx *c, const CgWork &w, void *x, size_t x_bytes, const void *b, d
             L.epi = ring.n == 1 ? EPI_CGUPDX : EPI_CGUPD;
             L.done = done;
             L.x = x;
-            L.p = p;
+            L.p = ps;
             L.r = r;
             L.red = rs;
             L.fin = FIN_RRNEW;
@@ -141,7 +166,10 @@ int cg_f64(wl_ctx *c, const CgWork &w, void *x, size_t x_bytes, const void *b, d
             }
             HIPCHK(launch_dslash(WL_F64, c->g, L, c->stream));
             // p = beta p + r, and x of a full ring (folded: with the convergence test and beta)
-            if (fold)
+            if (merged) {
+                if (it == n - 1)  // the state that the host looks at; else with the next hop
+                    HIPCHK(launch_cg_xpay_fold(c->g, PRing{{ps}, 1}, r, x, w.st, parts2, nhop, enqueued + it, c->stream));
+            } else if (fold)
                 HIPCHK(launch_cg_xpay_fold(c->g, ring, r, x, w.st, parts2, nhop, enqueued + it, c->stream));
             else
                 HIPCHK(launch_cg_xpay(WL_F64, c->g, ring, rs.slot, r, x, w.st, c->stream));

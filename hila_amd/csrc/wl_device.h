@@ -550,6 +550,36 @@ __device__ __forceinline__ double finish_order_sum(const double *partials, int n
     return out;
 }
 
+// The finish of iteration `it` (0-based) in the launch-folded CG (FIN_RRNEW,
+// conjugate_gradient.h:87-95): every workgroup adds the n partials of ||r||^2 in the finish
+// kernel's order and takes the same convergence decision and beta = rrnew / rr_it; workgroup 0
+// records the state (rrnew, iter, done; beta and rr, with rr_(it+1) in slot (it + 1) & 1, unless
+// converged).  False: the solve has ended, with this iteration or before.  The done flag is read
+// once per workgroup: workgroup 0 may set it meanwhile.  Contains barriers.
+__device__ __forceinline__ bool fold_rrnew(CgState *st, const double *parts, int n, int it, double &beta) {
+    __shared__ int ended;
+    if (threadIdx.x == 0) ended = st->done;
+    __syncthreads();
+    if (ended) return false;  // workgroup-uniform
+    const double s = finish_order_sum(parts, n);
+    const int iter = it + 1;
+    const bool conv = s < st->target_rr;
+    beta = s / st->rrb[it & 1];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->rrnew = s;
+        st->iter = iter;
+        if (conv) {
+            st->done = 1;
+        } else {
+            st->beta = beta;
+            st->rr = s;
+            st->rrb[(it + 1) & 1] = s;
+            if (iter >= st->maxiters) st->done = 2;
+        }
+    }
+    return !(conv || iter >= st->maxiters);
+}
+
 // Each workgroup of a reducing kernel stores its partial sum in partials[blockIdx.x]; a
 // one-workgroup finish kernel then adds them in workgroup order and applies the CG scalar
 // update (deterministic; no atomics).  A last-workgroup-finishes scheme would need a

@@ -75,6 +75,11 @@ struct DslashLaunch {
 // Kernel launchers (wl_dslash.hip / wl_blas.hip).  All enqueue on `s` and return hipError_t.
 hipError_t launch_dslash(int prec, const Geom &g, const DslashLaunch &L, hipStream_t s);
 
+// first hop of an iteration of the launch-folded CG in FP64 on the small-lattice kernel, with the
+// end of the iteration before: L.in the old p, L.r the residual, pnew = beta p + r (another
+// field), L.out = L.a H_+ pnew (odd); L.fold_parts, fold_n, fold_it as launch_cg_xpay_fold's
+hipError_t launch_dslash_xpay(const Geom &g, const DslashLaunch &L, void *pnew, hipStream_t s);
+
 // host AoS block <-> right-hand side j of an N-rhs field
 hipError_t launch_aos_to_soa(int prec, const Geom &g, const double *aos, void *planes, int N,
                              int j, hipStream_t s);
