@@ -360,6 +360,29 @@ int tile_rhs(const wl_ctx *c, int prec, int N) {
     return (N + groups - 1) / groups;
 }
 
+// Right-hand sides per workgroup of the direction-split kernel (wl_split.h) for N of them, 0: the
+// lane-per-site kernel.  A workgroup has one of the 256 CUs to itself, and loads its links and first
+// rhs, with nothing to overlap them, in the time of about two rhs: `cost`, of the grouping of the
+// rhs that takes the least, counts rhs of 128 lanes.  Up to 25/16 of the lanes that the sites fill it pays; hop,
+// us per rhs, lane per site / split (MI355X), and that ratio: 16^4 4 rhs 6.0 / 5.3 (1.50), 32^4 4 rhs
+// 83.6 / 80.1 (1.50), 12 rhs 80.9 / 61.2 (1.17), 24^3x48 12 rhs 51.7 / 46.3 (1.38), 8 rhs 50.8 / 49.3
+// (1.48), 6 rhs 51.6 / 52.6 (1.58), 4 rhs 55.9 / 58.2 (1.78), 48^3x24 12 rhs 114.7 / 102.1 (1.56),
+// 10x30x18x22 6 rhs 10.6 / 11.6 (2.2), 12^4 12 rhs 1.80 / 1.88 (2.1).  Not where the caller chose a
+// shape for the lane-per-site kernel, as wl_autotune does.
+int split_rhs(const wl_ctx *c, int prec, int N) {
+    const TileGeom &t = c->split;
+    if (prec != WL_F64 || !t.tiles) return 0;
+    if (c->rhs_block || c->rhs_launch || c->link_load || c->pipeline || !c->blk_auto || !c->lds_auto) return 0;
+    int best = N;
+    int64_t cost = INT64_MAX;
+    for (int groups = 1; groups <= std::max(1, N / 3); ++groups) {
+        const int per = (N + groups - 1) / groups;
+        const int64_t rounds = ((int64_t)t.tiles * groups + 255) / 256;
+        if (rounds * (per + 2) < cost) cost = rounds * (per + 2), best = per;
+    }
+    return cost * 256 * kSplitLanes * 16 <= (int64_t)c->g.vh * N * 25 ? best : 0;
+}
+
 int dslash_mr_all(wl_ctx *c, int prec, void *out, int out_par, const void *in, const void *xin,
                   double a, int sign, int epi, int N, const int *all_done, CgState *st, void *r,
                   int *pstride_out) {
@@ -369,27 +392,33 @@ int dslash_mr_all(wl_ctx *c, int prec, void *out, int out_par, const void *in, c
         if (rc) return rc;
     }
     if (!gauge_for(c, prec)) return fail(WL_E_STATE, "links of precision %d not prepared (ensure_gauge)", prec);
-    if (const int per = tile_rhs(c, prec, N)) {
+    const int tile = tile_rhs(c, prec, N), split = tile ? 0 : split_rhs(c, prec, N);
+    if (tile || split) {
+        const int slots = tile ? tile_slots(c->tile) : c->split.tiles;
         if (epi == EPI_AXPY_NORM || epi == EPI_CGUPD)
-            if (int rc = ensure_partials(c, (size_t)N * tile_slots(c->tile))) return rc;
+            if (int rc = ensure_partials(c, (size_t)N * slots)) return rc;
         MrLaunch L{};
         L.out = out;
         L.in = in;
         L.xin = xin;
         L.gauge = gauge_for(c, prec);
+        L.lf = link_format(c, prec);
         L.a = a;
         L.b = 1.0 + c->op_shift;
         L.out_par = out_par;
         L.sign = sign;
         L.epi = epi;
         L.NB = N;
-        L.NR = per;
+        L.NR = tile + split;
         L.all_done = all_done;
         L.st = st;
         L.r = r;
         L.partials = c->partials;
-        HIPCHK(launch_dslash_tile(c->g, c->tile, L, c->stream));
-        if (pstride_out) *pstride_out = tile_slots(c->tile);
+        if (tile)
+            HIPCHK(launch_dslash_tile(c->g, c->tile, L, c->stream));
+        else
+            HIPCHK(launch_dslash_split(c->g, c->split, L, c->stream));
+        if (pstride_out) *pstride_out = slots;
         return WL_OK;
     }
     const int nr = rhs_per_lane(c, prec, N);
@@ -552,6 +581,7 @@ extern "C" int wl_create(const int dims[4], int antiperiodic_t, int device, wl_c
     c->g.dir = dir_auto(c->g.vh);
     (void)set_chunk(c->g, -1);
     c->tile = tile_geom(c->g);
+    c->split = split_geom(c->g);
     DeviceGuard dg(device);
     int rc = WL_OK;
     // one partial-sum slot per workgroup of the largest grid (64-lane workgroups)

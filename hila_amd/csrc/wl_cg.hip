@@ -374,7 +374,7 @@ int BatchCG::prepare(wl_ctx *c, int N, int prec, bool mixed) {
         return rc;
     if (mixed && prec != WL_F64)
         if ((rc = work_field(c, W_Y, WL_F32, WL_EVEN, N, &f))) return rc;
-    const size_t rows = (size_t)std::max({nblocks(c->g), mr_segments(c->g), tile_slots(c->tile)});
+    const size_t rows = (size_t)std::max({nblocks(c->g), mr_segments(c->g), tile_slots(c->tile), c->split.tiles});
     if ((rc = ensure_partials(c, (size_t)N * rows))) return rc;
     return ensure_staging(c, (size_t)c->g.vh * 24 * sizeof(double));
 }
@@ -399,7 +399,7 @@ int BatchCG::reserve(wl_ctx *c, int N, int prec, bool mixed) {
         return rc;
     if (mixed && prec != WL_F64)
         if ((rc = work_field(c, W_Y, WL_F32, WL_EVEN, N, &f))) return rc;
-    const size_t rows = (size_t)std::max({nblocks(c->g), mr_segments(c->g), tile_slots(c->tile)});
+    const size_t rows = (size_t)std::max({nblocks(c->g), mr_segments(c->g), tile_slots(c->tile), c->split.tiles});
     if ((rc = ensure_partials(c, (size_t)N * rows))) return rc;
     // the gauge upload's staging (one direction of HILA's AoS links) is the larger one
     return ensure_staging(c, std::max((size_t)c->g.vh * 24, (size_t)c->V * 18) * sizeof(double));

@@ -211,6 +211,41 @@ inline TileGeom tile_geom(const Geom &g) {
 // partial sums per rhs of a launch: one for each wave of each tile
 inline int tile_slots(const TileGeom &t) { return t.tiles * (t.nt / 64); }
 hipError_t launch_dslash_tile(const Geom &g, const TileGeom &tg, const MrLaunch &L, hipStream_t s);
+
+// Tiles of the direction-split multi-rhs kernel (wl_split.h): as above, with at most kSplitLanes
+// output sites and kSplitSites staged ones, one for each lane of three directions.  The tiling with
+// the least work per site: lanes, idle ones too (about 45 clocks of a CU per rhs), and staged
+// sites (10).
+constexpr int kSplitLanes = 128;
+constexpr int kSplitSites = 3 * kSplitLanes;
+inline TileGeom split_geom(const Geom &g) {
+    const int Xh = g.L[0] / 2, Ly = g.L[1], Lz = g.L[2];
+    TileGeom best{};
+    if (g.stride > 1 << 24) return best;  // an rhs block is addressed with 32-bit byte offsets
+    double best_cost = 1e300;
+    for (int ty = 1; ty <= Ly && ty * Xh <= kSplitLanes; ++ty)
+        for (int tz = 1; tz <= Lz && ty * tz * Xh <= kSplitLanes; ++tz) {
+            const int stage = (ty * tz + 2 * ty + 2 * tz) * Xh;
+            if (stage > kSplitSites) continue;
+            TileGeom t{};
+            t.ty = ty;
+            t.tz = tz;
+            t.lanes = ty * tz * Xh;
+            t.nt = 4 * kSplitLanes;
+            t.ny = (Ly + ty - 1) / ty;
+            t.nz = (Lz + tz - 1) / tz;
+            t.tiles = t.ny * t.nz * g.L[3];
+            const double cost = (double)t.tiles * (45.0 * kSplitLanes + 10.0 * stage);
+            if (cost >= best_cost) continue;
+            best_cost = cost;
+            t.zs = 1;
+            for (int s = 1; s <= t.nz; ++s)
+                if (t.nz % s == 0 && (s == 1 || s * t.ny <= 8)) t.zs = s;
+            best = t;
+        }
+    return best;
+}
+hipError_t launch_dslash_split(const Geom &g, const TileGeom &tg, const MrLaunch &L, hipStream_t s);
 hipError_t launch_dslash_mr(int prec, const Geom &g, const MrLaunch &L, hipStream_t s);
 int mr_segments(const Geom &g);
 hipError_t launch_finish_mr(double *partials, int pstride, int n, int N, CgState *st,
@@ -272,7 +307,7 @@ struct wl_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     wl::Geom g{};
-    wl::TileGeom tile{};
+    wl::TileGeom tile{}, split{};
     int64_t V = 0;
     int antiperiodic = 1;
     void *gauge64 = nullptr;

@@ -40,8 +40,9 @@ __device__ __forceinline__ SiteAt site_at(int k) {
 // wanted needs no branch: the compiler counts the loads in flight between two points only where
 // no branch may skip some, and waits for all of them otherwise.
 typedef __amdgpu_buffer_rsrc_t Rsrc;
-__device__ __forceinline__ Rsrc rhs_block(const h2 *rhs, unsigned bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<h2 *>(rhs), 0, (int)bytes, 0x00020000);
+template <typename E>
+__device__ __forceinline__ Rsrc rhs_block(const E *rhs, unsigned bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<E *>(rhs), 0, (int)bytes, 0x00020000);
 }
 constexpr int kNT = 2;  // cache policy of streamed accesses: nontemporal
 
@@ -99,15 +100,49 @@ struct TileSite {
     bool st[kTileStage];
 };
 
-__host__ __device__ __forceinline__ TileSite tile_site(const Geom &g, const TileGeom &G, int p, int o, int tid, int nt) {
-    TileSite n;
-    // tile o: slab of zs z tiles, time slice, z tile of the slab, y tile
-    const int Xh = g.L[0] >> 1, Ly = g.L[1], Lz = g.L[2], Lt = g.L[3];
+// Time slice and first row of tile o: slab of zs z tiles, time slice, z tile of the slab, y tile.
+struct TileAt {
+    int t, y0, z0;
+};
+__host__ __device__ __forceinline__ TileAt tile_at(const Geom &g, const TileGeom &G, int o) {
     const int perslice = G.zs * G.ny;
-    const int slab = o / (perslice * Lt), os = o - slab * perslice * Lt;
+    const int slab = o / (perslice * g.L[3]), os = o - slab * perslice * g.L[3];
     const int t = os / perslice, q = os - t * perslice;
     const int zi = q / G.ny;
-    const int y0 = (q - zi * G.ny) * G.ty, z0 = (slab * G.zs + zi) * G.tz;
+    return {t, (q - zi * G.ny) * G.ty, (slab * G.zs + zi) * G.tz};
+}
+
+// The e-th site that tile c stages and its position; false past the last one.  The rows in
+// order: the one below in z, then each z with a row at either end in y, then the one above in z.
+__host__ __device__ __forceinline__ bool tile_staged(const Geom &g, const TileGeom &G, const TileAt &c, int e, int *k,
+                                                     int *pos) {
+    const int Xh = g.L[0] >> 1, Ly = g.L[1], Lz = g.L[2];
+    if (e >= (G.ty * G.tz + 2 * G.ty + 2 * G.tz) * Xh) return false;
+    int r = e / Xh;
+    const int x = e - r * Xh;
+    int rz = -1, ry = r;
+    if (r >= G.ty) {
+        r -= G.ty;
+        rz = r / (G.ty + 2);
+        ry = r - rz * (G.ty + 2) - 1;
+        if (rz >= G.tz) {
+            rz = G.tz;
+            ry = r - G.tz * (G.ty + 2);
+        }
+    }
+    int ys = c.y0 + ry, zs = c.z0 + rz;
+    ys += ys < 0 ? Ly : ys >= Ly ? -Ly : 0;
+    zs += zs < 0 ? Lz : zs >= Lz ? -Lz : 0;
+    *k = ((c.t * Lz + zs) * Ly + ys) * Xh + x;
+    *pos = ((rz + 1) * (G.ty + 2) + ry + 1) * Xh + x;
+    return true;
+}
+
+__host__ __device__ __forceinline__ TileSite tile_site(const Geom &g, const TileGeom &G, int p, int o, int tid, int nt) {
+    TileSite n;
+    const int Xh = g.L[0] >> 1, Ly = g.L[1], Lz = g.L[2], Lt = g.L[3];
+    const TileAt at = tile_at(g, G, o);
+    const int t = at.t, y0 = at.y0, z0 = at.z0;
     const int row = tid / Xh;
     int xh = tid - row * Xh;
     int zz = row / G.ty, yy = row - zz * G.ty;
@@ -129,30 +164,11 @@ __host__ __device__ __forceinline__ TileSite tile_site(const Geom &g, const Tile
     n.pos = (zz + 1) * n.pitch + (yy + 1) * Xh + xh;
     n.pxf = odd ? n.pos + xs : n.pos;
     n.pxb = odd ? n.pos : n.pos + xs;
-    // the rows to stage, in order: the one below in z, then each z with a row at either end in
-    // y, then the one above in z
-    const int nstage = (G.ty * G.tz + 2 * G.ty + 2 * G.tz) * Xh;
 #pragma unroll
     for (int i = 0; i < kTileStage; ++i) {
-        const int e = tid + i * nt;
-        n.st[i] = e < nstage;
-        int r = e / Xh;
-        const int x = e - r * Xh;
-        int rz = -1, ry = r;
-        if (r >= G.ty) {
-            r -= G.ty;
-            rz = r / (G.ty + 2);
-            ry = r - rz * (G.ty + 2) - 1;
-            if (rz >= G.tz) {
-                rz = G.tz;
-                ry = r - G.tz * (G.ty + 2);
-            }
-        }
-        int ys = y0 + ry, zs = z0 + rz;
-        ys += ys < 0 ? Ly : ys >= Ly ? -Ly : 0;
-        zs += zs < 0 ? Lz : zs >= Lz ? -Lz : 0;
-        n.ks[i] = n.st[i] ? ((t * Lz + zs) * Ly + ys) * Xh + x : k;
-        n.ps[i] = n.st[i] ? (rz + 1) * n.pitch + (ry + 1) * Xh + x : 0;  // 0: a corner, which nobody reads
+        n.ks[i] = k;
+        n.ps[i] = 0;  // a corner, which nobody reads
+        n.st[i] = tile_staged(g, G, at, tid + i * nt, &n.ks[i], &n.ps[i]);
     }
     return n;
 }
