@@ -496,6 +496,7 @@ int BatchCG::enqueue_chunk_body(int slot) {
     const int *all_done = c->flags_d;
     const int N = N_, prec = s_.prec;
     int rc;
+    static_assert(kChunk % 4 == 0, "a chunk ends with an empty ring");
     for (int it = 0; it < kChunk; ++it) {
         int ps = 0;
         const int q = it % ring_.n;
