@@ -152,7 +152,7 @@ template <int SIGN, int EPI, int LF>
 __global__ __launch_bounds__(kSplitThreads, 2) void k_dslash_split(RbArgs<double> A, TileGeom G) {
     // staged components [component][position]; partial sums [component][of three directions][site]
     extern __shared__ __align__(16) unsigned char split_smem[];
-    __shared__ double red[2][kSplitThreads / 64];
+    __shared__ double red[2][kSplitWaves];
     constexpr bool norms = EPI == EPI_AXPY_NORM || EPI == EPI_CGUPD;
     u32x4 *stage = reinterpret_cast<u32x4 *>(split_smem);
     cx<double> *part = reinterpret_cast<cx<double> *>(split_smem + sizeof(u32x4) * 12 * kSplitSites);
@@ -201,7 +201,7 @@ __global__ __launch_bounds__(kSplitThreads, 2) void k_dslash_split(RbArgs<double
     // the wave sums of rhs jj, in red[b]
     auto store_norm = [&](int jj, int b) {
         double s = 0;
-        for (int i = 0; i < kSplitThreads / 64; ++i) s += red[b][i];
+        for (int i = 0; i < kSplitWaves; ++i) s += red[b][i];
         A.partials[(size_t)jj * A.pstride + o] = s;
     };
     int last = -1;
