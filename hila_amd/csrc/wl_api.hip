@@ -343,44 +343,13 @@ Geom mr_geom(const wl_ctx *c, int prec, int nb, int nr, bool lds_links) {
     return g;
 }
 
-// Right-hand sides per workgroup of the LDS-tiled kernel (wl_tile.h) for N of them, 0: the
-// lane-per-site kernel.  A tile's links and first rhs are loaded with nothing to overlap them
-// (31 us of a launch on 32^4, 14 us for each rhs), so it takes six: M in FP16, us per rhs, lane
-// per site / tiled (MI355X): 24^3x48 4 rhs 30.8 / 32.4, 6 rhs 29.7 / 28.6, 12 rhs 28.9 / 25.2;
-// 32^4 12 rhs 45.0 / 35.5; 16^3x32 12 rhs 5.8 / 5.2.  The rhs are split into as many groups, of
-// three at least, as make 1024 workgroups (20^4 with 320 tiles, 12 rhs: 7.35 in one group, 6.89
-// in four; 24^4 with 864: 14.4 and 13.2 in two); with fewer than 256 tiles (16^4, 12 rhs: 3.06 / 3.15)
-// and where tiles waste more than one lane in eight (48^3x24, rows of 24: 119 / 121) it does not
-// pay.  Not where the caller chose a shape for the lane-per-site kernel, as wl_autotune does.
-int tile_rhs(const wl_ctx *c, int prec, int N) {
-    const TileGeom &t = c->tile;
-    if (prec != WL_F16 || N < 6 || t.tiles < 256 || (int64_t)t.tiles * t.nt * 8 > (int64_t)c->g.vh * 9) return 0;
-    if (c->rhs_block || c->rhs_launch || c->link_load || c->pipeline || !c->blk_auto || !c->lds_auto) return 0;
-    const int groups = std::min((1024 + t.tiles - 1) / t.tiles, N / 3);
-    return (N + groups - 1) / groups;
-}
-
-// Right-hand sides per workgroup of the direction-split kernel (wl_split.h) for N of them, 0: the
-// lane-per-site kernel.  A workgroup has one of the 256 CUs to itself, and loads its links and first
-// rhs, with nothing to overlap them, in the time of about two rhs: `cost`, of the grouping of the
-// rhs that takes the least, counts rhs of 128 lanes.  Up to 25/16 of the lanes that the sites fill it pays; hop,
-// us per rhs, lane per site / split (MI355X), and that ratio: 16^4 4 rhs 6.0 / 5.3 (1.50), 32^4 4 rhs
-// 83.6 / 80.1 (1.50), 12 rhs 80.9 / 61.2 (1.17), 24^3x48 12 rhs 51.7 / 46.3 (1.38), 8 rhs 50.8 / 49.3
-// (1.48), 6 rhs 51.6 / 52.6 (1.58), 4 rhs 55.9 / 58.2 (1.78), 48^3x24 12 rhs 114.7 / 102.1 (1.56),
-// 10x30x18x22 6 rhs 10.6 / 11.6 (2.2), 12^4 12 rhs 1.80 / 1.88 (2.1).  Not where the caller chose a
-// shape for the lane-per-site kernel, as wl_autotune does.
-int split_rhs(const wl_ctx *c, int prec, int N) {
-    const TileGeom &t = c->split;
-    if (prec != WL_F64 || !t.tiles) return 0;
-    if (c->rhs_block || c->rhs_launch || c->link_load || c->pipeline || !c->blk_auto || !c->lds_auto) return 0;
-    int best = N;
-    int64_t cost = INT64_MAX;
-    for (int groups = 1; groups <= std::max(1, N / 3); ++groups) {
-        const int per = (N + groups - 1) / groups;
-        const int64_t rounds = ((int64_t)t.tiles * groups + 255) / 256;
-        if (rounds * (per + 2) < cost) cost = rounds * (per + 2), best = per;
-    }
-    return cost * 256 * kSplitLanes * 16 <= (int64_t)c->g.vh * N * 25 ? best : 0;
+MrChoice mr_choice(const wl_ctx *c, int prec, int N) {
+    const bool always = c->tiled_hop == 1;
+    if (c->tiled_hop >= 0 && prec == WL_F16)
+        if (const int per = tile_rhs(c->tile, c->g.vh, N, always)) return {HOP_TILE, per};
+    if (c->tiled_hop >= 0 && prec == WL_F64)
+        if (const int per = split_rhs(c->split, c->g.vh, N, always)) return {HOP_SPLIT, per};
+    return {HOP_LANE, 0};
 }
 
 int dslash_mr_all(wl_ctx *c, int prec, void *out, int out_par, const void *in, const void *xin,
@@ -392,8 +361,9 @@ int dslash_mr_all(wl_ctx *c, int prec, void *out, int out_par, const void *in, c
         if (rc) return rc;
     }
     if (!gauge_for(c, prec)) return fail(WL_E_STATE, "links of precision %d not prepared (ensure_gauge)", prec);
-    const int tile = tile_rhs(c, prec, N), split = tile ? 0 : split_rhs(c, prec, N);
-    if (tile || split) {
+    const MrChoice how = mr_choice(c, prec, N);
+    if (how.kernel != HOP_LANE) {
+        const bool tile = how.kernel == HOP_TILE;
         const int slots = tile ? tile_slots(c->tile) : c->split.tiles;
         if (epi == EPI_AXPY_NORM || epi == EPI_CGUPD)
             if (int rc = ensure_partials(c, (size_t)N * slots)) return rc;
@@ -409,7 +379,7 @@ int dslash_mr_all(wl_ctx *c, int prec, void *out, int out_par, const void *in, c
         L.sign = sign;
         L.epi = epi;
         L.NB = N;
-        L.NR = tile + split;
+        L.NR = how.per;
         L.all_done = all_done;
         L.st = st;
         L.r = r;
@@ -921,6 +891,11 @@ extern "C" int wl_set_option(wl_ctx *c, int option, int value) {
         if (value != 0 && value != 1) return fail(WL_E_ARG, "pipeline option must be 0 or 1");
         c->pipeline = value;
         return WL_OK;
+    case WL_OPT_TILED_HOP:
+        if (value < -1 || value > 1)
+            return fail(WL_E_ARG, "tiled hop option must be -1 (never), 0 (automatic) or 1 (wherever there are tiles)");
+        c->tiled_hop = value;
+        return WL_OK;
     case WL_OPT_LINK_ROWS: {
         if (value != 2 && value != 3) return fail(WL_E_ARG, "link rows must be 3 (full links) or 2 (two-row links)");
         const int prev = c->link_rows;
@@ -960,6 +935,7 @@ extern "C" int wl_get_option(const wl_ctx *c, int option, int *value) {
     case WL_OPT_LDS_RESERVE: *value = lds_reserve_of(c); return WL_OK;
     case WL_OPT_GRAPHS: *value = c->use_graphs ? 1 : 0; return WL_OK;
     case WL_OPT_PIPELINE: *value = c->pipeline; return WL_OK;
+    case WL_OPT_TILED_HOP: *value = c->tiled_hop; return WL_OK;
     case WL_OPT_LINK_ROWS: *value = c->link_rows; return WL_OK;
     case WL_OPT_CG_PERSISTENT: *value = c->cg_persistent; return WL_OK;
     case WL_OPT_SMALL_HOP: *value = c->small_hop; return WL_OK;
@@ -968,22 +944,31 @@ extern "C" int wl_get_option(const wl_ctx *c, int option, int *value) {
     }
 }
 
+extern "C" int wl_hop_kernel(const wl_ctx *c, int prec, int nrhs, int *kernel) {
+    if (!c || !kernel) return fail(WL_E_ARG, "null argument");
+    if (prec != WL_F64 && prec != WL_F32 && prec != WL_F16) return fail(WL_E_NOTIMPL, "precision %d", prec);
+    if (nrhs < 1 || nrhs > 64) return fail(WL_E_ARG, "nrhs %d out of range 1..64", nrhs);
+    *kernel = mr_choice(c, prec, nrhs).kernel;
+    return WL_OK;
+}
+
 // ================================================================== autotuner ===========
 
 namespace {
 
 // A tuning holds for one lattice size, precision and rhs count, and for the link format and
-// link-load and pipelining modes it was timed with (they change the kernels' speed).
+// link-load, pipelining and tiled-hop modes it was timed with (they change the kernels' speed).
 struct TuneKey {
-    int L[4], prec, nrhs, link_format, link_load, pipeline;
+    int L[4], prec, nrhs, link_format, link_load, pipeline, tiled_hop;
     bool operator<(const TuneKey &o) const {
-        return std::tie(L[0], L[1], L[2], L[3], prec, nrhs, link_format, link_load, pipeline) <
-               std::tie(o.L[0], o.L[1], o.L[2], o.L[3], o.prec, o.nrhs, o.link_format, o.link_load, o.pipeline);
+        return std::tie(L[0], L[1], L[2], L[3], prec, nrhs, link_format, link_load, pipeline, tiled_hop) <
+               std::tie(o.L[0], o.L[1], o.L[2], o.L[3], o.prec, o.nrhs, o.link_format, o.link_load, o.pipeline,
+                        o.tiled_hop);
     }
 };
 TuneKey tune_key(const wl_ctx *c, int prec, int nrhs) {
     return TuneKey{{c->g.L[0], c->g.L[1], c->g.L[2], c->g.L[3]}, prec, nrhs, link_format(c, prec), c->link_load,
-                   c->pipeline};
+                   c->pipeline, c->tiled_hop};
 }
 std::mutex g_tune_mu;
 std::map<TuneKey, wl_tune_result> g_tuned;
@@ -1104,7 +1089,10 @@ extern "C" int wl_autotune(wl_ctx *c, int prec, int nrhs, wl_tune_result *out) {
     if (saved.lds_reserve > 0) reserves.push_back(saved.lds_reserve);
     const int nr_cap = prec == WL_F64 ? 2 : 4;
     static const int launches[] = {1, 2, 4, 6, 12, 16, 24, 32, 48, 64};
-    for (int nr = 1; nr <= std::min(nr_cap, nrhs); nr *= 2) {
+    // a launch that takes a tiled kernel has no shape to choose: the default configuration only
+    const bool tiled = mr_choice(c, prec, nrhs).kernel != HOP_LANE;
+    if (tiled) count = 1;
+    for (int nr = 1; nr <= std::min(nr_cap, nrhs) && !tiled; nr *= 2) {
         std::vector<int> nls;  // effective rhs per launch (multiples of nr, or all)
         for (int want : launches) {
             if (want > nrhs) want = nrhs;
@@ -1152,7 +1140,7 @@ extern "C" int wl_autotune(wl_ctx *c, int prec, int nrhs, wl_tune_result *out) {
     cleanup();
     std::sort(t_best.begin(), t_best.end());
     std::sort(t_def.begin(), t_def.end());
-    if (t_def[1] <= t_best[1]) {
+    if (tiled || t_def[1] <= t_best[1]) {
         def.us_per_rhs = t_def[1];
         best = def;
     } else {

@@ -120,6 +120,8 @@ int rhs_per_lane(const wl_ctx *c, int prec, int N);
 // rhs per launch for a requested count: a multiple of nr (at least nr), at most N
 int rhs_per_launch_of(int want, int nr, int N);
 int rhs_per_launch(const wl_ctx *c, int nr, int N);
+// the kernel that dslash_mr_all takes for N right-hand sides
+MrChoice mr_choice(const wl_ctx *c, int prec, int N);
 // out = a H_sign in (+ epilogue) for N right-hand sides; per-rhs partial sums land in
 // c->partials rows, *pstride_out apart.
 int dslash_mr_all(wl_ctx *c, int prec, void *out, int out_par, const void *in, const void *xin,

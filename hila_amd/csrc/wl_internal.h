@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstddef>
 #include <cstdint>
 #include <mutex>
@@ -246,6 +247,52 @@ inline TileGeom split_geom(const Geom &g) {
     return best;
 }
 hipError_t launch_dslash_split(const Geom &g, const TileGeom &tg, const MrLaunch &L, hipStream_t s);
+
+// Which kernel applies the multi-rhs hopping term, and how many right-hand sides a workgroup of it
+// takes.  It follows from the lattice, the precision, the rhs count and WL_OPT_TILED_HOP alone: the
+// kernels add in different orders, and neither launch-shape options nor the autotuner, which goes
+// by time, may change a result.
+enum HopKernel : int { HOP_LANE = 0, HOP_TILE = 1, HOP_SPLIT = 2 };
+struct MrChoice {
+    HopKernel kernel;
+    int per;
+};
+
+// Right-hand sides per workgroup of the LDS-tiled kernel (wl_tile.h) for N of them in FP16, 0: the
+// lane-per-site kernel.  A tile's links and first rhs are loaded with nothing to overlap them
+// (31 us of a launch on 32^4, 14 us for each rhs), so it takes six: M in FP16, us per rhs, lane
+// per site / tiled (MI355X): 24^3x48 4 rhs 30.8 / 32.4, 6 rhs 29.7 / 28.6, 12 rhs 28.9 / 25.2;
+// 32^4 12 rhs 45.0 / 35.5; 16^3x32 12 rhs 5.8 / 5.2.  The rhs are split into as many groups, of
+// three at least, as make 1024 workgroups (20^4 with 320 tiles, 12 rhs: 7.35 in one group, 6.89
+// in four; 24^4 with 864: 14.4 and 13.2 in two); with fewer than 256 tiles (16^4, 12 rhs: 3.06 / 3.15)
+// and where tiles waste more than one lane in eight (48^3x24, rows of 24: 119 / 121) it does not
+// pay.  always: wherever the lattice has tiles (WL_OPT_TILED_HOP = 1).
+inline int tile_rhs(const TileGeom &t, int vh, int N, bool always) {
+    if (!t.tiles) return 0;
+    if (!always && (N < 6 || t.tiles < 256 || (int64_t)t.tiles * t.nt * 8 > (int64_t)vh * 9)) return 0;
+    const int groups = std::max(1, std::min((1024 + t.tiles - 1) / t.tiles, N / 3));
+    return (N + groups - 1) / groups;
+}
+
+// Right-hand sides per workgroup of the direction-split kernel (wl_split.h) for N of them in FP64, 0:
+// the lane-per-site kernel.  A workgroup has one of the 256 CUs to itself, and loads its links and first
+// rhs, with nothing to overlap them, in the time of about two rhs: `cost`, of the grouping of the
+// rhs that takes the least, counts rhs of 128 lanes.  Up to 25/16 of the lanes that the sites fill it pays; hop,
+// us per rhs, lane per site / split (MI355X), and that ratio: 16^4 4 rhs 6.0 / 5.3 (1.50), 32^4 4 rhs
+// 83.6 / 80.1 (1.50), 12 rhs 80.9 / 61.2 (1.17), 24^3x48 12 rhs 51.7 / 46.3 (1.38), 8 rhs 50.8 / 49.3
+// (1.48), 6 rhs 51.6 / 52.6 (1.58), 4 rhs 55.9 / 58.2 (1.78), 48^3x24 12 rhs 114.7 / 102.1 (1.56),
+// 10x30x18x22 6 rhs 10.6 / 11.6 (2.2), 12^4 12 rhs 1.80 / 1.88 (2.1).
+inline int split_rhs(const TileGeom &t, int vh, int N, bool always) {
+    if (!t.tiles) return 0;
+    int best = N;
+    int64_t cost = INT64_MAX;
+    for (int groups = 1; groups <= std::max(1, N / 3); ++groups) {
+        const int per = (N + groups - 1) / groups;
+        const int64_t rounds = ((int64_t)t.tiles * groups + 255) / 256;
+        if (rounds * (per + 2) < cost) cost = rounds * (per + 2), best = per;
+    }
+    return always || cost * 256 * kSplitLanes * 16 <= (int64_t)vh * N * 25 ? best : 0;
+}
 hipError_t launch_dslash_mr(int prec, const Geom &g, const MrLaunch &L, hipStream_t s);
 int mr_segments(const Geom &g);
 hipError_t launch_finish_mr(double *partials, int pstride, int n, int N, CgState *st,
@@ -354,6 +401,7 @@ struct wl_ctx {
     int link_load = 0;                 // multi-rhs links: 0 automatic, 1 cached, 2 nontemporal, 3 LDS
     bool use_graphs = false;           // batched CG: replay each chunk from a captured HIP graph
     int pipeline = 0;                  // multi-rhs hops: 0 pipelined where possible, 1 never
+    int tiled_hop = 0;                 // WL_OPT_TILED_HOP: 0 automatic, -1 never, 1 wherever there are tiles
     int cg_persistent = 0;             // single-rhs FP64 CG in one launch: 1 yes (where the
                                        // launch fits), 0 (default: kernel by kernel, launch-
                                        // folded on small lattices) or -1 kernel by kernel

@@ -16,9 +16,9 @@
 // budget.
 //
 // A request is solved exactly as the blocking wl_cg_solve / wl_cg_solve_mixed of the same
-// right-hand sides on a fresh context would solve it: the kernels and their launch shapes
-// depend only on the lattice size, the precision and the rhs count, so a result does not
-// depend on what else is being served.
+// right-hand sides on a fresh context, with the launch shape that wl_autotune remembers for them
+// if it was called, would solve it: the kernels and their launch shapes depend only on the lattice
+// size, the precision and the rhs count, so a result does not depend on what else is being served.
 
 #include <algorithm>
 #include <atomic>
@@ -694,7 +694,8 @@ extern "C" int wl_server_info_get(wl_server *S, wl_server_info *info) {
 
 extern "C" int wl_server_set_option(wl_server *S, int option, int value) {
     if (!S) return fail(WL_E_ARG, "null server");
-    if (option < WL_OPT_TRAVERSAL_CHUNK || option > WL_OPT_LINK_ROWS) return fail(WL_E_ARG, "unknown option %d", option);
+    if ((option < WL_OPT_TRAVERSAL_CHUNK || option > WL_OPT_LINK_ROWS) && option != WL_OPT_TILED_HOP)
+        return fail(WL_E_ARG, "unknown option %d", option);
     std::lock_guard<std::mutex> lk(S->mu);
     if (S->submitted) return fail(WL_E_STATE, "server options must be set before the first submission");
     S->slot_opts.emplace_back(option, value);

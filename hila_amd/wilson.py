@@ -30,7 +30,7 @@ EVEN, ODD = 1, 2
 F64, F32, F16 = 0, 1, 2
 OPT_TRAVERSAL_CHUNK, OPT_BLOCK, OPT_RHS_BLOCK, OPT_RHS_LAUNCH, OPT_PLANE_PAD, OPT_LINK_LOAD = 1, 2, 3, 4, 5, 6
 OPT_LDS_RESERVE, OPT_GRAPHS, OPT_PIPELINE, OPT_LINK_ROWS, OPT_CG_PERSISTENT, OPT_SMALL_HOP = 7, 8, 9, 10, 11, 12
-OPT_BLOCK_KRYLOV = 13
+OPT_BLOCK_KRYLOV, OPT_TILED_HOP = 13, 14
 
 EXPORTED_SYMBOLS = [
     "wl_version", "wl_last_error", "wl_create", "wl_destroy", "wl_sync", "wl_volume",
@@ -38,7 +38,7 @@ EXPORTED_SYMBOLS = [
     "wl_field_download", "wl_field_zero", "wl_field_copy", "wl_field_norm2", "wl_dslash_eo", "wl_meo_apply",
     "wl_cg_solve", "wl_cg_solve_mixed", "wl_set_option", "wl_get_option", "wl_time_op", "wl_gen_gauge", "wl_gen_spinor", "wl_gen_point",
     "wl_server_create", "wl_server_submit", "wl_server_wait", "wl_server_info_get", "wl_server_destroy",
-    "wl_host_alloc", "wl_host_free", "wl_autotune", "wl_server_set_option",
+    "wl_host_alloc", "wl_host_free", "wl_autotune", "wl_hop_kernel", "wl_server_set_option",
     "wl_gauge_download", "wl_config_header", "wl_config_read", "wl_config_write",
     "wl_hasenbusch_apply", "wl_cg_solve_ex", "wl_mre_guess", "wl_field_copy_rhs",
     "wl_fermion_force", "wl_momentum_upload", "wl_momentum_download", "wl_fermion_force_step",
@@ -151,6 +151,7 @@ def lib():
         L.wl_server_destroy.argtypes = [vp]
         L.wl_host_alloc.argtypes = [C.c_size_t, C.POINTER(vp)]
         L.wl_host_free.argtypes = [vp]
+        L.wl_hop_kernel.argtypes = [vp, i, i, C.POINTER(i)]
         L.wl_autotune.argtypes = [vp, i, i, C.POINTER(TuneResult)]
         L.wl_server_set_option.argtypes = [vp, i, i]
         L.wl_gauge_download.argtypes = [vp, C.POINTER(vp)]
@@ -291,6 +292,13 @@ class Lattice:
     def get_option(self, option):
         v = C.c_int(0)
         check(lib().wl_get_option(self.handle, int(option), C.byref(v)))
+        return v.value
+
+    def hop_kernel(self, prec, nrhs):
+        """The kernel that applies the hopping term to nrhs right-hand sides stored in prec: 0 one
+        lane per site, 1 LDS tiles, 2 LDS tiles split by direction (wl_hop_kernel)."""
+        v = C.c_int(0)
+        check(lib().wl_hop_kernel(self.handle, int(prec), int(nrhs), C.byref(v)))
         return v.value
 
     def autotune(self, prec, nrhs):

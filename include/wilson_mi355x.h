@@ -324,7 +324,19 @@ int wl_hasenbusch2_force_step(wl_ctx *ctx, const wl_field *chi, wl_field *psi, d
  *       kernel by kernel.  Results are identical either way.
  *   WL_OPT_PIPELINE  multi-rhs kernel: 0 (default) = software-pipelined hops where the
  *       registers allow (FP32 and FP16 storage, up to 2 rhs per lane); 1 = never.
- * Results do not depend on these options; only the speed does.
+ * Results do not depend on these options, bit for bit, except that WL_OPT_RHS_BLOCK,
+ * WL_OPT_LINK_LOAD = 3 and WL_OPT_PIPELINE run other compiled forms of the one-lane-per-site kernel,
+ * which agree to rounding.  These three, WL_OPT_BLOCK, WL_OPT_RHS_LAUNCH and WL_OPT_LDS_RESERVE
+ * shape launches of one lane per site; the LDS-tiled kernels (WL_OPT_TILED_HOP) have a shape of
+ * their own, and no option but that one changes which kernel a launch takes.
+ * The following choose between ways to compute a result:
+ *   WL_OPT_TILED_HOP  hopping launches of several right-hand sides: 0 (default) = LDS-tiled
+ *       kernels where they are the faster ones, which the lattice, the precision and the rhs count
+ *       alone decide (FP16 storage from 6 rhs; FP64 from 4, with more of them the fewer sites fill
+ *       a tile; wl_hop_kernel); -1 = one lane per site always; 1 = LDS tiles wherever the lattice
+ *       has them, FP32 storage excepted.  FP64 results agree to rounding
+ *       (the hops are summed in another order); FP16 operators agree bit for bit, and solves with
+ *       an FP16 inner precision to rounding (||.||^2 is summed in another order).
  *   WL_OPT_LINK_ROWS  3 (default): the FP64 and FP32 hopping kernels read all 9 entries of
  *       every link.  2: they read rows 0 and 1 and rebuild row 2 as conj(row 0 x row 1), 96
  *       instead of 144 bytes per FP64 link (a third less link traffic).  Allowed only for
@@ -378,10 +390,15 @@ enum {
     WL_OPT_LINK_ROWS = 10,
     WL_OPT_CG_PERSISTENT = 11,
     WL_OPT_SMALL_HOP = 12,
-    WL_OPT_BLOCK_KRYLOV = 13
+    WL_OPT_BLOCK_KRYLOV = 13,
+    WL_OPT_TILED_HOP = 14
 };
 int wl_set_option(wl_ctx *ctx, int option, int value);
 int wl_get_option(const wl_ctx *ctx, int option, int *value);
+/* The kernel that applies the hopping term to nrhs right-hand sides stored in prec
+ * (WL_OPT_TILED_HOP): 0 one lane per site (or, for one rhs, the small-lattice kernel of
+ * WL_OPT_SMALL_HOP), 1 LDS tiles (FP16), 2 LDS tiles split by direction (FP64). */
+int wl_hop_kernel(const wl_ctx *ctx, int prec, int nrhs, int *kernel);
 
 /* Autotuner of the multi-rhs hopping kernel (no counterpart in HILA).  For nrhs right-hand
  * sides at precision prec it times the hopping term on scratch fields of this context for
@@ -390,11 +407,13 @@ int wl_get_option(const wl_ctx *ctx, int option, int *value);
  * and sets WL_OPT_RHS_BLOCK, WL_OPT_RHS_LAUNCH and WL_OPT_BLOCK to the fastest (in FP64 and
  * FP32 also WL_OPT_LDS_RESERVE: automatic, i.e. the occupancy cap where it applies, or none).
  * The choice is timed again against the default configuration, which is kept unless the choice
- * is faster.  The choice is
+ * is faster.  Where the launch takes an LDS-tiled kernel (wl_hop_kernel) there is no shape to
+ * choose: the default configuration is timed and kept.  The choice is
  * remembered per (lattice size, precision, nrhs, link format WL_OPT_LINK_ROWS, WL_OPT_LINK_LOAD,
- * WL_OPT_PIPELINE) for the life of the process, so that later calls, and other contexts of the
- * same size and options, take the same configuration without timing again (results then do
- * not depend on timing noise).  The gauge field must be uploaded. */
+ * WL_OPT_PIPELINE, WL_OPT_TILED_HOP) for the life of the process, so that later calls, and other
+ * contexts of the same size and options, take the same configuration without timing again.  A
+ * choice that sets WL_OPT_RHS_BLOCK changes results by rounding, as the option does; no choice
+ * changes which kernel a launch takes.  The gauge field must be uploaded. */
 typedef struct wl_tune_result {
     int rhs_block;            /* 0 in all three: the default configuration was fastest      */
     int rhs_launch;
