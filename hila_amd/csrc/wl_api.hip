@@ -343,10 +343,10 @@ Geom mr_geom(const wl_ctx *c, int prec, int nb, int nr, bool lds_links) {
     return g;
 }
 
-MrChoice mr_choice(const wl_ctx *c, int prec, int N) {
+MrChoice mr_choice(const wl_ctx *c, int prec, int N, bool alone) {
     const bool always = c->tiled_hop == 1;
     if (c->tiled_hop >= 0 && prec == WL_F16)
-        if (const int per = tile_rhs(c->tile, c->g.vh, N, always)) return {HOP_TILE, per};
+        if (const int per = tile_rhs(c->tile, c->g.vh, N, alone, always)) return {HOP_TILE, per};
     if (c->tiled_hop >= 0 && prec == WL_F64)
         if (const int per = split_rhs(c->split, c->g.vh, N, always)) return {HOP_SPLIT, per};
     return {HOP_LANE, 0};
@@ -354,14 +354,14 @@ MrChoice mr_choice(const wl_ctx *c, int prec, int N) {
 
 int dslash_mr_all(wl_ctx *c, int prec, void *out, int out_par, const void *in, const void *xin,
                   double a, int sign, int epi, int N, const int *all_done, CgState *st, void *r,
-                  int *pstride_out) {
+                  int *pstride_out, bool alone) {
     const int pstride = mr_segments(c->g);
     if (epi == EPI_AXPY_NORM || epi == EPI_CGUPD) {
         int rc = ensure_partials(c, (size_t)N * pstride);
         if (rc) return rc;
     }
     if (!gauge_for(c, prec)) return fail(WL_E_STATE, "links of precision %d not prepared (ensure_gauge)", prec);
-    const MrChoice how = mr_choice(c, prec, N);
+    const MrChoice how = mr_choice(c, prec, N, alone);
     if (how.kernel != HOP_LANE) {
         const bool tile = how.kernel == HOP_TILE;
         const int slots = tile ? tile_slots(c->tile) : c->split.tiles;
@@ -760,7 +760,7 @@ extern "C" int wl_dslash_eo(wl_ctx *c, wl_field *out, const wl_field *in, double
         return dslash_one(c, in->prec, out->data, out_par, in->data, nullptr, -kappa, sign, EPI_SET,
                           nullptr, FIN_NONE);
     return dslash_mr_all(c, in->prec, out->data, out_par, in->data, nullptr, -kappa, sign, EPI_SET,
-                         in->nrhs, nullptr, nullptr, nullptr, nullptr);
+                         in->nrhs, nullptr, nullptr, nullptr, nullptr, true);
 }
 
 namespace {
@@ -944,11 +944,12 @@ extern "C" int wl_get_option(const wl_ctx *c, int option, int *value) {
     }
 }
 
-extern "C" int wl_hop_kernel(const wl_ctx *c, int prec, int nrhs, int *kernel) {
+extern "C" int wl_hop_kernel(const wl_ctx *c, int what, int prec, int nrhs, int *kernel) {
     if (!c || !kernel) return fail(WL_E_ARG, "null argument");
+    if (what != 0 && what != 1) return fail(WL_E_ARG, "what must be 0 (hopping term) or 1 (M and solves)");
     if (prec != WL_F64 && prec != WL_F32 && prec != WL_F16) return fail(WL_E_NOTIMPL, "precision %d", prec);
     if (nrhs < 1 || nrhs > 64) return fail(WL_E_ARG, "nrhs %d out of range 1..64", nrhs);
-    *kernel = mr_choice(c, prec, nrhs).kernel;
+    *kernel = mr_choice(c, prec, nrhs, what == 0).kernel;
     return WL_OK;
 }
 
@@ -979,7 +980,7 @@ int time_hop_mr(wl_ctx *c, int prec, void *out, const void *in, int N, int iters
     for (int i = 0; i < 2 + iters; ++i) {
         if (i == 2) HIPCHK(hipEventRecord(e0, c->stream));
         if (int rc = dslash_mr_all(c, prec, out, 1, in, nullptr, -0.125, 1, EPI_SET, N, nullptr, nullptr, nullptr,
-                                   nullptr))
+                                   nullptr, true))
             return rc;
     }
     HIPCHK(hipEventRecord(e1, c->stream));
@@ -1090,7 +1091,7 @@ extern "C" int wl_autotune(wl_ctx *c, int prec, int nrhs, wl_tune_result *out) {
     const int nr_cap = prec == WL_F64 ? 2 : 4;
     static const int launches[] = {1, 2, 4, 6, 12, 16, 24, 32, 48, 64};
     // a launch that takes a tiled kernel has no shape to choose: the default configuration only
-    const bool tiled = mr_choice(c, prec, nrhs).kernel != HOP_LANE;
+    const bool tiled = mr_choice(c, prec, nrhs, true).kernel != HOP_LANE;
     if (tiled) count = 1;
     for (int nr = 1; nr <= std::min(nr_cap, nrhs) && !tiled; nr *= 2) {
         std::vector<int> nls;  // effective rhs per launch (multiples of nr, or all)

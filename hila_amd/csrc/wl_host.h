@@ -121,12 +121,12 @@ int rhs_per_lane(const wl_ctx *c, int prec, int N);
 int rhs_per_launch_of(int want, int nr, int N);
 int rhs_per_launch(const wl_ctx *c, int nr, int N);
 // the kernel that dslash_mr_all takes for N right-hand sides
-MrChoice mr_choice(const wl_ctx *c, int prec, int N);
+MrChoice mr_choice(const wl_ctx *c, int prec, int N, bool alone);
 // out = a H_sign in (+ epilogue) for N right-hand sides; per-rhs partial sums land in
-// c->partials rows, *pstride_out apart.
+// c->partials rows, *pstride_out apart.  alone: a hopping term by itself (tile_rhs).
 int dslash_mr_all(wl_ctx *c, int prec, void *out, int out_par, const void *in, const void *xin,
                   double a, int sign, int epi, int N, const int *all_done, CgState *st, void *r,
-                  int *pstride_out);
+                  int *pstride_out, bool alone = false);
 // M_s for N right-hand sides (even fields) through the odd work field t
 int meo_mr(wl_ctx *c, int prec, void *out, const void *in, void *t, double kappa, int sign,
            int epi2, int N, const int *all_done, CgState *st, int *pstride_out);

@@ -259,19 +259,49 @@ struct MrChoice {
 };
 
 // Right-hand sides per workgroup of the LDS-tiled kernel (wl_tile.h) for N of them in FP16, 0: the
-// lane-per-site kernel.  A tile's links and first rhs are loaded with nothing to overlap them
-// (31 us of a launch on 32^4, 14 us for each rhs), so it takes six: M in FP16, us per rhs, lane
-// per site / tiled (MI355X): 24^3x48 4 rhs 30.8 / 32.4, 6 rhs 29.7 / 28.6, 12 rhs 28.9 / 25.2;
-// 32^4 12 rhs 45.0 / 35.5; 16^3x32 12 rhs 5.8 / 5.2.  The rhs are split into as many groups, of
-// three at least, as make 1024 workgroups (20^4 with 320 tiles, 12 rhs: 7.35 in one group, 6.89
-// in four; 24^4 with 864: 14.4 and 13.2 in two); with fewer than 256 tiles (16^4, 12 rhs: 3.06 / 3.15)
-// and where tiles waste more than one lane in eight (48^3x24, rows of 24: 119 / 121) it does not
-// pay.  always: wherever the lattice has tiles (WL_OPT_TILED_HOP = 1).
-inline int tile_rhs(const TileGeom &t, int vh, int N, bool always) {
+// lane-per-site kernel.  alone: the hopping term by itself, not inside M or a solve; always:
+// wherever the lattice has tiles (WL_OPT_TILED_HOP = 1).
+//
+// A tile loads its links and first rhs, with nothing to overlap them, in the time of about two rhs;
+// a CU holds 8 of its waves; and of the bytes per lane about half are staged, in runs of ty or
+// ty + 2 rows that end inside lines of 8 sites (16-byte vectors) unless the rows are aligned.  So
+// `cost`, of the grouping of the rhs that takes the least, is rhs of lanes per rhs of sites, 1 at
+// best; one or two rounds of workgroups that leave over an eighth of the slots idle are no choice
+// (24^4, 864 tiles for 512 slots, M with 12 rhs: 14.8 us per rhs in one group, 13.2 in two).  Up to
+// 1.4 the tiles pay in M and the solves, and up to 1.7 where the spinors do not stay in the caches
+// (256 MB of Infinity Cache), which help the lane-per-site kernel more.  The hopping
+// term alone touches no other field, so its spinors stay there up to 3 to 3.5 x 2^20 site-rhs, and
+// until then the lane-per-site kernel is the faster one.  Lane per site / tiled (MI355X), M, us per rhs:
+//   cost up to 1.4: 16^3x32 12 rhs (1.25) 5.52 / 5.01, 16^3x64 6 rhs (1.25) 12.4 / 11.3, 32^4 12 rhs
+//   (1.17) 46.0 / 36.6; above: 16^3x32 6 rhs (1.56) 6.43 / 6.48, 20^4 6 rhs (2.2) 7.45 / 8.40, 18^3x36
+//   12 rhs (1.53) 9.4 / 10.3, 10x26x24x32 12 rhs (1.85) 8.90 / 10.6;
+//   from 1.5 x 2^20 site-rhs: 24^3x48 12 rhs (1.43) 29.2 / 25.4, 8 rhs (1.53) 29.2 / 27.1, 6 rhs (1.63)
+//   28.7 / 29.4; above 1.7: 26^4 12 rhs (2.0) level, 22^3x44 12 rhs (2.1) 22.7 / 24.2;
+// a solve, ms per iteration: 16^3x32 12 rhs 0.234 / 0.217, 24^3x48 8 rhs 0.782 / 0.733, 20^4 6 rhs 0.162 /
+//   0.177, 10x26x24x32 6 rhs 0.194 / 0.242, 8x26x10x64 12 rhs 0.230 / 0.260;
+// the hopping term alone, us per rhs: 16^3x32 12 rhs (0.75 x 2^20) 2.21 / 2.30, 24^3x48 8 rhs (2.5) 10.6 /
+//   13.0, 12 rhs (3.8) 13.5 / 11.4, 32^4 6 rhs (3) 22.7 / 18.0.
+// Not tried with fewer than 256 tiles or 6 rhs, or where tiles waste more than one lane in eight
+// (48^3x24, rows of 24: 119 / 121).
+inline int tile_rhs(const TileGeom &t, int vh, int N, bool alone, bool always) {
     if (!t.tiles) return 0;
     if (!always && (N < 6 || t.tiles < 256 || (int64_t)t.tiles * t.nt * 8 > (int64_t)vh * 9)) return 0;
-    const int groups = std::max(1, std::min((1024 + t.tiles - 1) / t.tiles, N / 3));
-    return (N + groups - 1) / groups;
+    const int slots = 256 * (8 / (t.nt / 64));
+    int per = N;
+    int64_t least = INT64_MAX;
+    for (int groups = 1; groups <= std::max(1, N / 3); ++groups) {
+        const int p = (N + groups - 1) / groups, n = (N + p - 1) / p;
+        const int64_t rounds = ((int64_t)t.tiles * n + slots - 1) / slots;
+        const bool idle = rounds <= 2 && rounds * slots * 8 > (int64_t)t.tiles * n * 9;
+        if ((always || !idle) && rounds * (p + 2) < least) least = rounds * (p + 2), per = p;
+    }
+    if (always || least == INT64_MAX) return always ? per : 0;
+    const int Xh = t.lanes / (t.ty * t.tz), broken = 8 - std::min(Xh & -Xh, 8);
+    const double staged = t.tz * ((t.ty + 2) * Xh + broken) + 2 * (t.ty * Xh + broken);
+    const double sites = (double)vh * N;
+    const double cost = (double)least * slots * t.nt / sites * (2 + staged / t.lanes) / 4;
+    constexpr double M = 1 << 20;
+    return (cost <= 1.41 && (!alone || sites >= 3 * M)) || (cost <= 1.72 && sites >= (alone ? 3.5 : 1.5) * M) ? per : 0;
 }
 
 // Right-hand sides per workgroup of the direction-split kernel (wl_split.h) for N of them in FP64, 0:
@@ -281,7 +311,8 @@ inline int tile_rhs(const TileGeom &t, int vh, int N, bool always) {
 // us per rhs, lane per site / split (MI355X), and that ratio: 16^4 4 rhs 6.0 / 5.3 (1.50), 32^4 4 rhs
 // 83.6 / 80.1 (1.50), 12 rhs 80.9 / 61.2 (1.17), 24^3x48 12 rhs 51.7 / 46.3 (1.38), 8 rhs 50.8 / 49.3
 // (1.48), 6 rhs 51.6 / 52.6 (1.58), 4 rhs 55.9 / 58.2 (1.78), 48^3x24 12 rhs 114.7 / 102.1 (1.56),
-// 10x30x18x22 6 rhs 10.6 / 11.6 (2.2), 12^4 12 rhs 1.80 / 1.88 (2.1).
+// 10x30x18x22 6 rhs 10.6 / 11.6 (2.2), 12^4 12 rhs 1.80 / 1.88 (2.1).  What the rule gets wrong, by
+// 2 to 6%: 12^3x96 8 rhs (1.48) 10.9 / 11.6, 14x18x14x64 6 rhs (1.55), 24^3x96 6 rhs (1.51).
 inline int split_rhs(const TileGeom &t, int vh, int N, bool always) {
     if (!t.tiles) return 0;
     int best = N;

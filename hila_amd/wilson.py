@@ -151,7 +151,7 @@ def lib():
         L.wl_server_destroy.argtypes = [vp]
         L.wl_host_alloc.argtypes = [C.c_size_t, C.POINTER(vp)]
         L.wl_host_free.argtypes = [vp]
-        L.wl_hop_kernel.argtypes = [vp, i, i, C.POINTER(i)]
+        L.wl_hop_kernel.argtypes = [vp, i, i, i, C.POINTER(i)]
         L.wl_autotune.argtypes = [vp, i, i, C.POINTER(TuneResult)]
         L.wl_server_set_option.argtypes = [vp, i, i]
         L.wl_gauge_download.argtypes = [vp, C.POINTER(vp)]
@@ -294,11 +294,12 @@ class Lattice:
         check(lib().wl_get_option(self.handle, int(option), C.byref(v)))
         return v.value
 
-    def hop_kernel(self, prec, nrhs):
-        """The kernel that applies the hopping term to nrhs right-hand sides stored in prec: 0 one
-        lane per site, 1 LDS tiles, 2 LDS tiles split by direction (wl_hop_kernel)."""
+    def hop_kernel(self, prec, nrhs, what="M"):
+        """The kernel that applies the hopping term to nrhs right-hand sides stored in prec, in M and
+        the solves or by itself (what="hop"): 0 one lane per site, 1 LDS tiles, 2 LDS tiles split by
+        direction (wl_hop_kernel)."""
         v = C.c_int(0)
-        check(lib().wl_hop_kernel(self.handle, int(prec), int(nrhs), C.byref(v)))
+        check(lib().wl_hop_kernel(self.handle, {"hop": 0, "M": 1}[what], int(prec), int(nrhs), C.byref(v)))
         return v.value
 
     def autotune(self, prec, nrhs):

@@ -332,8 +332,8 @@ int wl_hasenbusch2_force_step(wl_ctx *ctx, const wl_field *chi, wl_field *psi, d
  * The following choose between ways to compute a result:
  *   WL_OPT_TILED_HOP  hopping launches of several right-hand sides: 0 (default) = LDS-tiled
  *       kernels where they are the faster ones, which the lattice, the precision and the rhs count
- *       alone decide (FP16 storage from 6 rhs; FP64 from 4, with more of them the fewer sites fill
- *       a tile; wl_hop_kernel); -1 = one lane per site always; 1 = LDS tiles wherever the lattice
+ *       alone decide (FP16 storage from 6 rhs where the tiles fill the device; FP64 from 4, with
+ *       more of them the fewer sites fill a tile; wl_hop_kernel); -1 = one lane per site always; 1 = LDS tiles wherever the lattice
  *       has them, FP32 storage excepted.  FP64 results agree to rounding
  *       (the hops are summed in another order); FP16 operators agree bit for bit, and solves with
  *       an FP16 inner precision to rounding (||.||^2 is summed in another order).
@@ -396,9 +396,10 @@ enum {
 int wl_set_option(wl_ctx *ctx, int option, int value);
 int wl_get_option(const wl_ctx *ctx, int option, int *value);
 /* The kernel that applies the hopping term to nrhs right-hand sides stored in prec
- * (WL_OPT_TILED_HOP): 0 one lane per site (or, for one rhs, the small-lattice kernel of
- * WL_OPT_SMALL_HOP), 1 LDS tiles (FP16), 2 LDS tiles split by direction (FP64). */
-int wl_hop_kernel(const wl_ctx *ctx, int prec, int nrhs, int *kernel);
+ * (WL_OPT_TILED_HOP), by itself (what = 0, wl_dslash_eo) or in M and the solves (what = 1): 0 one
+ * lane per site (or, for one rhs, the small-lattice kernel of WL_OPT_SMALL_HOP), 1 LDS tiles
+ * (FP16), 2 LDS tiles split by direction (FP64). */
+int wl_hop_kernel(const wl_ctx *ctx, int what, int prec, int nrhs, int *kernel);
 
 /* Autotuner of the multi-rhs hopping kernel (no counterpart in HILA).  For nrhs right-hand
  * sides at precision prec it times the hopping term on scratch fields of this context for
