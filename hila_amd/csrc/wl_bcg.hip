@@ -40,7 +40,7 @@ namespace {
 
 constexpr int kBcgMax = 24;    // right-hand sides of one block
 
-// The FP32 inner solution of the mixed solvers (BatchCG's y, folded into x by k_fold_mr) is
+// The FP32 inner solution of a mixed solve (folded into x by k_fold_mr) is
 // laid out as the FP64 solution is, one complex number per component: unpacked FP32.
 struct f32u {};
 constexpr int kF32Unpacked = 100;  // its precision code in launch_bcombo
@@ -491,12 +491,12 @@ int cg_block(wl_ctx *c, void *x, const void *b, int N, const CgSpec &spec, wl_cg
         }
         const bool update = est_done || (mixed && (dropped || it - it_update >= spec.update_every));
         if (update) {
-            if (mixed) HIPCHK(launch_fold_mr(c->g, x, B.Y->data, c->st_mr, 1, N, nullptr, S));
+            if (mixed) HIPCHK(launch_fold_mr(c->g, x, B.Y->data, N, S));
             if ((rc = restart(false))) return rc;
         }
     }
     if (!converged) {  // maxiters: the final true residual
-        if (mixed) HIPCHK(launch_fold_mr(c->g, x, B.Y->data, c->st_mr, 1, N, nullptr, S));
+        if (mixed) HIPCHK(launch_fold_mr(c->g, x, B.Y->data, N, S));
         Mat G64;
         if ((rc = B.true_residual(G64))) return rc;
         for (int j = 0; j < N; ++j)

@@ -312,7 +312,7 @@ inline int tile_rhs(const TileGeom &t, int vh, int N, bool alone, bool always) {
 // 83.6 / 80.1 (1.50), 12 rhs 80.9 / 61.2 (1.17), 24^3x48 12 rhs 51.7 / 46.3 (1.38), 8 rhs 50.8 / 49.3
 // (1.48), 6 rhs 51.6 / 52.6 (1.58), 4 rhs 55.9 / 58.2 (1.78), 48^3x24 12 rhs 114.7 / 102.1 (1.56),
 // 10x30x18x22 6 rhs 10.6 / 11.6 (2.2), 12^4 12 rhs 1.80 / 1.88 (2.1).  What the rule gets wrong, by
-// 2 to 6%: 12^3x96 8 rhs (1.48) 10.9 / 11.6, 14x18x14x64 6 rhs (1.55), 24^3x96 6 rhs (1.51).
+// 2 to 6%: 12^3x96 8 rhs (1.48) 9.9 / 10.5, 14x18x14x64 6 rhs (1.55), 24^3x96 6 rhs (1.51).
 inline int split_rhs(const TileGeom &t, int vh, int N, bool always) {
     if (!t.tiles) return 0;
     int best = N;
@@ -349,9 +349,8 @@ hipError_t launch_batch_sync(CgState *st, int N, int mixed, int *flags, const in
 hipError_t launch_zero_rhs(const Geom &g, void *x, int j, hipStream_t s);
 // *flag = 1 if every one of the N rhs has converged (done == 1), else 0
 hipError_t launch_all_converged(const CgState *st, int N, int *flag, hipStream_t s);
-// x_j += y_j, y_j = 0 (x FP64, y FP32) for rhs taking a reliable update, or all with all != 0
-hipError_t launch_fold_mr(const Geom &g, void *x, void *y, const CgState *st, int all, int N, const int *gate,
-                          hipStream_t s);
+// x_j += y_j, y_j = 0 (x FP64, y FP32) for every rhs
+hipError_t launch_fold_mr(const Geom &g, void *x, void *y, int N, hipStream_t s);
 
 // one-workgroup kernel: sum nparts partials in order, apply `fin` (skipped when *done != 0)
 hipError_t launch_finish(const RedArgs &ra, int nparts, int fin, const int *done, hipStream_t s);

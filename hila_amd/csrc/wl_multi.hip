@@ -147,13 +147,11 @@ __global__ __launch_bounds__(kBlock) void k_flush_mr(RingArgs<T> ring, cx<double
     if (n > 1) st_site<T>(ring.p[0] + off, S, k, pv);
 }
 
-// Fold the inner solution into the FP64 one: x_j += y_j, y_j = 0, for the rhs that take a
-// reliable update (done 3 or 4), or for every rhs with all != 0.  Skipped when *gate != 0.
-__global__ __launch_bounds__(kBlock) void k_fold_mr(cx<double> *__restrict__ x, cx<float> *__restrict__ y,
-                                                    const CgState *st, int all, int vh, int S, const int *gate) {
-    if (gate && *gate) return;
+// Fold the inner solution of a block solve into the FP64 one: x_j += y_j, y_j = 0.
+__global__ __launch_bounds__(kBlock) void k_fold_mr(cx<double> *__restrict__ x, cx<float> *__restrict__ y, int vh,
+                                                    int S) {
     const int k = blockIdx.x * kBlock + threadIdx.x, j = blockIdx.y;
-    if (k >= vh || !(all || st[j].done == 3 || st[j].done == 4)) return;
+    if (k >= vh) return;
     const size_t off = (size_t)j * 12 * S;
 #pragma unroll
     for (int c = 0; c < 12; ++c) {
@@ -376,10 +374,9 @@ hipError_t launch_batch_sync(CgState *st, int N, int mixed, int *flags, const in
     return hipGetLastError();
 }
 
-hipError_t launch_fold_mr(const Geom &g, void *x, void *y, const CgState *st, int all, int N, const int *gate,
-                          hipStream_t s) {
-    hipLaunchKernelGGL(k_fold_mr, dim3(nblocks(g), N), dim3(kBlock), 0, s, (cx<double> *)x, (cx<float> *)y, st, all,
-                       g.vh, g.stride, gate);
+hipError_t launch_fold_mr(const Geom &g, void *x, void *y, int N, hipStream_t s) {
+    hipLaunchKernelGGL(k_fold_mr, dim3(nblocks(g), N), dim3(kBlock), 0, s, (cx<double> *)x, (cx<float> *)y, g.vh,
+                       g.stride);
     return hipGetLastError();
 }
 
