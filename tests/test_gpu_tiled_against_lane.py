@@ -113,3 +113,29 @@ def test_solve(dims, precision):
     for s, t in zip(*counts):
         assert abs(s - t) <= (max(1, t // 10) if precision == "f16" else 1)
     lat.close()
+
+
+@pytest.mark.parametrize("precision,n", [("f64", 4), ("f32", 4), ("f16", 8)])
+def test_captured_chunks(precision, n):
+    """Chunks with the tiled kernels (144 KB of dynamic LDS in FP64) captured into a HIP graph and
+    replayed, with eager work between the solves, give the bits of the eager solve."""
+    lat = _lattice((16, 16, 16, 32))
+    prec = {"f64": W.F64, "f32": W.F32, "f16": W.F16}[precision]
+    assert lat.hop_kernel(W.F64, n) == 2 and lat.hop_kernel(prec, n) == {W.F64: 2, W.F32: 0, W.F16: 1}[prec]
+    D = W.Dirac_Wilson_evenodd(0.124, lat)
+    cg = W.CG(D, 1e-9, 2000, precision=precision, delta=1e-1)
+    b, x, tmp = W.Field(lat, nrhs=n), W.Field(lat, nrhs=n), W.Field(lat, nrhs=n)
+    for j in range(n):
+        b.upload(W.gen_spinor(lat.dims, 60 + j), j)
+    x.zero()
+    eager = cg.apply(b, x, raise_on_noconv=True)
+    ref = [x.download(j) for j in range(n)]
+    lat.set_option(W.OPT_GRAPHS, 1)
+    for _ in range(3):
+        D.apply(b, tmp)
+        lat.sync()
+        x.zero()
+        st = cg.apply(b, x)
+        assert [(s["iterations"], s["true_resid"]) for s in st] == [(s["iterations"], s["true_resid"]) for s in eager]
+        assert all(np.array_equal(x.download(j), ref[j]) for j in range(n))
+    lat.close()
