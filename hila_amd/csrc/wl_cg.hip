@@ -32,8 +32,8 @@ bool cg_fold(const wl_ctx *c, const CgWork &w) {
 // look costs the device about 25 us of waiting, an iteration enqueued past the end 4 to 7 launches
 // that return at once, 1.5 to 3 us each.  So after the first kChunk: up to four iterations short
 // of where ||r||^2, going down as it did since the last look, would stop the solve, and then to
-// one past that.  Against a look every kChunk iterations: 8^4 (56 of them) 1642 -> 1587 us, the
-// solve of a force step on 16^3x32 5.70 -> 5.63 ms, large lattices level.
+// one past that.  Against a look every kChunk iterations: 8^4 3-5% less, the solve of a force step
+// on 16^3x32 5.70 -> 5.63 ms, large lattices level.
 class Pace {
     double log_rr_ = 0, rate_ = 0;  // ln ||r||^2 at the last look, its decline per iteration
     int iter_ = -1;
@@ -53,8 +53,9 @@ class Pace {
 };
 
 // The kernel-by-kernel FP64 CG on work memory w.  An iteration is M p with ||Dp||^2 partials,
-// the finish of alpha, M^dag Dp fused with the x, r update and ||r||^2 partials, the finish of
-// rrnew (convergence, beta) and p = beta p + r: seven launches.  Folded (cg_fold), the alpha
+// the finish of alpha, M^dag Dp fused with the r update and ||r||^2 partials, the finish of
+// rrnew (convergence, beta) and p = beta p + r, with the x update where the ring of search
+// directions is full (PRing; without a ring, x is updated with r): seven launches.  Folded (cg_fold), the alpha
 // finish moves into the update pass and the rrnew finish into p = beta p + r: five launches,
 // the same sums in the same order, so the same bits.  With the small-lattice kernel (g.dir) the
 // latter move on into the next iteration's first hop: four launches (k_dslash_dir_xpay).

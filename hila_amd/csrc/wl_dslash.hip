@@ -146,9 +146,10 @@ __global__ __launch_bounds__(256) void k_dslash_dir(DslashArgs<R> A) {
 // the end of iteration `it` folded in: its finish (fold_rrnew) and p = beta p_old + r, which every
 // wave forms at the neighbours it gathers, from p_old and r.  The x wave's neighbours include the
 // even site with the lane's own index, whose p it stores.  So an iteration is four launches, not
-// five: on 8^4 this one takes 7.0 us and replaces
-// 5.0 (hop) + 4.1 (p) and the gap between them; a solve of 56 iterations 1555 -> 1413 us, on 16^4
-// 3.81 -> 3.77 ms.
+// five: on 8^4 this one takes 7.0 us and replaces 5.0 (hop) + 4.1 (p) and the gap between them.
+// A solve of 51 iterations, with the paced looks of the host: 1610 -> 1465 us; 12^4 2.07 -> 1.92 ms,
+// 16^4 3.81 -> 3.77.  It holds two neighbours of p and of r: 256 VGPRs and 32 AGPRs, one wave per
+// SIMD, which is why 16^4, the largest lattice that takes it, gains least.
 // A.in: p_old, A.r: r (read), A.fold_*: the partials of ||r||^2 and `it`.
 template <int LF>
 __global__ __launch_bounds__(256) void k_dslash_dir_xpay(DslashArgs<double> A, cx<double> *__restrict__ pnew) {

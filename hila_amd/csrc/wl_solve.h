@@ -25,7 +25,9 @@
 
 namespace wl {
 
-constexpr int kChunk = 8;  // iterations per chunk (one host check each)
+// Iterations per chunk of the batched solves (one host check each), and until the first look of the
+// single-rhs ones, which pace the later looks themselves.
+constexpr int kChunk = 8;
 
 struct CgSpec {
     double kappa = 0.125;

@@ -13,7 +13,7 @@
 // gains little.)  Here 52 x (2 + the staged rows per output row) + 288 / rhs bytes pass it, about
 // 240, and the rest is read from LDS at twice the rate.  32^4, 12 rhs, us per rhs (MI355X): 21.3
 // lane per site, 16.6 here, of which arithmetic is 64% and 1.13 GB a launch miss the L2 (at
-// 5.6 TB/s; 0.81 GB are needed); M 46.8 and 37.0, on 24^3x48 28.9 and 25.2.
+// 5.6 TB/s; 0.81 GB are needed); M 46.0 and 36.6, on 24^3x48 29.2 and 25.4.
 #pragma once
 
 #include "wl_rb.h"
@@ -35,8 +35,8 @@ __device__ __forceinline__ SiteAt site_at(int k) {
     return {(unsigned)(k >> 6) * 3072u + (unsigned)(k & 63) * 16u, (unsigned)k * 4u};
 }
 
-// An rhs block as a buffer of `bytes` bytes (under 4 GB, tile_geom; 0: reads give 0, writes are
-// dropped, and neither reaches memory).  One offset register an address, and a load that is not
+// An rhs block as a buffer of `bytes` bytes (under 4 GB, tile_geom; 0: reads, whose results nobody
+// uses, mostly give 0 without reaching memory, and would lie inside the block if they did).  One offset register an address, and a load that is not
 // wanted needs no branch: the compiler counts the loads in flight between two points only where
 // no branch may skip some, and waits for all of them otherwise.
 typedef __amdgpu_buffer_rsrc_t Rsrc;

@@ -316,9 +316,10 @@ int wl_hasenbusch2_force_step(wl_ctx *ctx, const wl_field *chi, wl_field *psi, d
  *       more rhs, or of two or more on lattices of 2^17 sites per parity or more, which reserve
  *       32 KB per 64 lanes (at most 5 workgroups per CU), and FP32 launches of four or more
  *       rhs at 3-4 per lane on lattices of 2^17 sites per parity or more, 24 KB (6); both,
- *       unless WL_OPT_BLOCK is set, in 64-lane workgroups).  The
- *       kernels use no LDS; the reservation caps how many workgroups share a CU, i.e. the
- *       sites in flight, whose neighbour spinors must fit the caches to be reused.
+ *       unless WL_OPT_BLOCK is set, in 64-lane workgroups).  The one-lane-per-site
+ *       kernels use no LDS of their own (unless WL_OPT_LINK_LOAD = 3); the reservation caps how
+ *       many workgroups share a CU, i.e. the sites in flight, whose neighbour spinors must fit
+ *       the caches to be reused.
  *   WL_OPT_GRAPHS  1: the batched CG (nrhs > 1, FP16 inner, the server) captures each chunk
  *       of iterations into a HIP graph once per solve and replays it; 0 (default): launches
  *       kernel by kernel.  Results are identical either way.
@@ -350,10 +351,11 @@ int wl_hasenbusch2_force_step(wl_ctx *ctx, const wl_field *chi, wl_field *psi, d
  *       1 = the whole solve -- source norm, initial residual, every iteration and the final
  *       true residual -- runs as one cooperative launch whose workgroups meet at grid
  *       barriers, with no host round trip inside the solve; -1 = kernel by kernel, seven
- *       launches per iteration, with the host checking convergence every 8 iterations; 0
- *       (default) = kernel by kernel, and on lattices of up to 2^15 sites per parity with
- *       the two finish kernels of an iteration folded into the kernels after them (five
- *       launches).  On MI355X the grid barriers of the one-launch solve (an L2 write-back and
+ *       launches per iteration, with the host checking convergence at intervals that it paces
+ *       by the decline of the residual; 0 (default) = kernel by kernel, and on lattices of up
+ *       to 2^15 sites per parity with the two finish kernels of an iteration folded into the
+ *       kernels after them and, with the small-lattice hopping kernel, the next search
+ *       direction into the next iteration's first hop (five and four launches).  On MI355X the grid barriers of the one-launch solve (an L2 write-back and
  *       invalidate per XCD each) cost more than the kernel boundaries they replace, at every
  *       lattice size.
  *       Both give the same solution, bit for bit: the persistent launch runs the same per-site
