@@ -33,7 +33,9 @@ bool cg_fold(const wl_ctx *c, const CgWork &w) {
 // that return at once, 1.5 to 3 us each.  So after the first kChunk: up to four iterations short
 // of where ||r||^2, going down as it did since the last look, would stop the solve, and then to
 // one past that.  Against a look every kChunk iterations: 8^4 3-5% less, the solve of a force step
-// on 16^3x32 5.70 -> 5.63 ms, large lattices level.
+// on 16^3x32 5.70 -> 5.63 ms, large lattices level; with reliable updates every 5 or 6 iterations (8^4, FP32,
+// delta 0.1), where a prediction that is short by one costs a look, 2% more.  Never less than kChunk at a
+// time, or three quarters of the way instead of four short: 1-9% more on 8^4.
 class Pace {
     double log_rr_ = 0, rate_ = 0;  // ln ||r||^2 at the last look, its decline per iteration
     int iter_ = -1;
